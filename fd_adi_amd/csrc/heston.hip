@@ -17,8 +17,8 @@
 // derivative at both variance ends, d2/dv2 Von Neumann 0 at v=0 and the
 // second-order backward row (with its -2 band entry, folded) at vmax.
 //
-// Sweeps.  A spot sweep is one workgroup per (option, tile of NL variance
-// columns); a variance sweep one workgroup per (option, tile of NL spot
+// Sweeps.  A spot sweep gives each workgroup (option, tile of NL variance
+// columns) pairs, one or, for wide tiles, one after another; a variance sweep one workgroup per (option, tile of NL spot
 // rows).  The tile's right-hand side is formed (fusing every explicit term of
 // the stage) straight into LDS, the NL tridiagonal lines are solved in LDS,
 // and the stage output (fusing the next stage's explicit term) is written
@@ -277,6 +277,57 @@ __device__ void affine_scan(const double *cM, const double *cE, double *cIn) {
   }
 }
 
+// The same for four-column tiles without a scan through LDS: the value entering
+// this thread's chunk of its line, given the chunk's map y -> E + M y and 0
+// entering the line's first chunk (REV: its last; the maps are applied from
+// the last chunk down).  A wave holds 16 chunks of each line, lane = chunk * 4
+// + line: it scans them across lanes, leaves the map of all of them in
+// tot[waves][4], and after one barrier composes the carry entering the wave
+// from the waves before it.  One barrier instead of three: a single option is
+// bound by latency, and its solve runs on four-column tiles.  Calls that
+// follow one another without a barrier in between use different `tot`s.
+template <int CTRL>
+__device__ __forceinline__ void map_level(double &M, double &E) {
+  const double Mp = dpp_or<CTRL, 0xF>(M, 1.0), Ep = dpp_or<CTRL, 0xF>(E, 0.0);
+  E = E + M * Ep;
+  M = M * Mp;
+}
+__device__ __forceinline__ void map_level_from(double &M, double &E, int src, bool take) {
+  const double Mp = __shfl(M, src, 64), Ep = __shfl(E, src, 64);
+  E = take ? E + M * Ep : E;
+  M = take ? M * Mp : M;
+}
+
+template <int THREADS, bool REV>
+__device__ __forceinline__ double quad_carry(double M, double E, double2 *tot) {
+  constexpr int NW = THREADS / 64;
+  const int lane = threadIdx.x % 64, wave = threadIdx.x / 64, line = lane % 4, row = lane / 16;
+  // inclusive scan over the wave's chunks: within rows of 16 lanes by DPP
+  // (row_shl / row_shr by 4 and 8 lanes), then across rows from a row's last
+  // chunk in scan order
+  map_level<REV ? 0x104 : 0x114>(M, E);
+  map_level<REV ? 0x108 : 0x118>(M, E);
+  const int end = REV ? line : 12 + line;
+  map_level_from(M, E, (REV ? row | 1 : row & ~1) * 16 + end, (row & 1) == (REV ? 0 : 1));
+  map_level_from(M, E, (REV ? 32 : 16) + end, REV ? row < 2 : row >= 2);
+  const bool first = REV ? lane >= 60 : lane < 4;
+  if (REV ? lane < 4 : lane >= 60) tot[wave * 4 + line] = make_double2(M, E);
+  // the map of the chunks before this one
+  const int prev = (REV ? lane + 4 : lane - 4) & 63;
+  const double Mp = __shfl(M, prev, 64), Ep = __shfl(E, prev, 64);
+  __syncthreads();
+  double c = 0.0;
+#pragma unroll
+  for (int q = 0; q < NW - 1; ++q) {
+    const int w = REV ? NW - 1 - q : q;
+    if (REV ? w > wave : w < wave) {
+      const double2 t = tot[w * 4 + line];
+      c = t.y + t.x * c;
+    }
+  }
+  return first ? c : Ep + Mp * c;
+}
+
 // ---- spot sweep ---------------------------------------------------------------
 // One 128-byte row of per-node spot coefficients, built from the spot table
 // with the boundary handling folded in:
@@ -336,26 +387,16 @@ __device__ __forceinline__ ColOp col_op(double c, double gsub, double gmid, doub
 }
 
 // A state row at this lane's column j: columns j-1, j, j+1 (clamped to the
-// grid) and j-2 on the grid's last column (0 elsewhere).
-struct Row4 {
-  double l, c, r, m2;
+// grid).
+struct Row3 {
+  double l, c, r;
 };
 
-struct LaneCols {  // this lane's column indices within a row (clamped)
-  unsigned jm, jc, jp, jm2, jx;
-  bool last;
+// This lane's columns of a tile, as byte offsets within a state row.
+struct LaneCols {
+  unsigned jcb, jxb;  // column j and the edge column, clamped to the grid
+  bool last, ok;      // j is the grid's last column (or clamped to it) / inside the grid
 };
-
-__device__ __forceinline__ Row4 load_row4(const double *__restrict__ f, unsigned rowoff,
-                                          const LaneCols &lc) {
-  const double *p = f + rowoff;
-  Row4 w;
-  w.l = p[lc.jm];
-  w.c = p[lc.jc];
-  w.r = p[lc.jp];
-  w.m2 = lc.last ? p[lc.jm2] : 0.0;
-  return w;
-}
 
 // A row as loaded for the window: column j and this lane's edge column jx
 // (j - 1 on the tile's first lane, j + 1 on its last, j elsewhere).  The
@@ -368,26 +409,47 @@ struct Raw2 {
   double e, c;
 };
 
-__device__ __forceinline__ Raw2 load_raw2(const double *__restrict__ f, unsigned rowoff,
-                                          const LaneCols &lc) {
-  const double *p = f + rowoff;
-  return Raw2{p[lc.jx], p[lc.jc]};
+// An option's state (or pivots) as a buffer of nS * nv doubles addressed by
+// 32-bit byte offsets: a read past it (also at a negative offset, which wraps
+// far beyond its end) gives 0 and a store past it is dropped, so rows outside
+// the grid need no clamping and no lane masks.
+using Buf = __amdgpu_buffer_rsrc_t;
+typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ Buf buf_of(const double *p, unsigned bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<double *>(p), 0, (int)bytes, 0x00027000);
+}
+__device__ __forceinline__ double buf_load(Buf b, unsigned off) {
+  const u32x2 v = __builtin_amdgcn_raw_buffer_load_b64(b, (int)off, 0, 0);
+  return __hiloint2double((int)v.y, (int)v.x);
+}
+__device__ __forceinline__ void buf_store(Buf b, unsigned off, double x) {
+  const u32x2 v = {(unsigned)__double2loint(x), (unsigned)__double2hiint(x)};
+  __builtin_amdgcn_raw_buffer_store_b64(v, b, (int)off, 0, 0);
 }
 
-// A double at a 32-bit byte offset from a work-group-uniform base: the global
-// access takes the scalar base + 32-bit lane offset form, with no 64-bit
-// address arithmetic per lane.
-__device__ __forceinline__ double load_at(const double *__restrict__ base, unsigned byte_off) {
-  return *reinterpret_cast<const double *>(reinterpret_cast<const char *>(base) + byte_off);
-}
-__device__ __forceinline__ void store_at(double *__restrict__ base, unsigned byte_off, double v) {
-  *reinterpret_cast<double *>(reinterpret_cast<char *>(base) + byte_off) = v;
+// The row at byte offset rowb (row * nv * 8).
+__device__ __forceinline__ Raw2 load_raw2(Buf f, unsigned rowb, const LaneCols &lc) {
+  return Raw2{buf_load(f, rowb + lc.jxb), buf_load(f, rowb + lc.jcb)};
 }
 
-// load_raw2 with the row given as a byte offset (row * nv * 8).
-__device__ __forceinline__ Raw2 load_raw2_at(const double *__restrict__ f, unsigned rowb,
-                                             const LaneCols &lc) {
-  return Raw2{load_at(f, rowb + lc.jx * 8u), load_at(f, rowb + lc.jc * 8u)};
+// 16 bytes per lane from `src` into LDS at dst + 16 * lane (dst uniform over
+// the wave), without passing through registers; lds_loads_done() waits for
+// this wave's, a barrier after it for everyone's.
+__device__ __forceinline__ void load_lds16(const double *src, double *dst) {
+  __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)src,
+                                   (__attribute__((address_space(3))) void *)dst, 16, 0, 0);
+}
+__device__ __forceinline__ void lds_loads_done() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+
+// 1 / d by two Newton steps from the hardware estimate (relative error
+// 2^-23, then 2^-46 and below 2^-90 before the last rounding): as the IEEE
+// division, whose special cases v_div_fixup supplies, at half its
+// instructions.
+__device__ __forceinline__ double recip(double d) {
+  double r = __builtin_amdgcn_rcp(d);
+  r = __builtin_fma(r, __builtin_fma(-d, r, 1.0), r);
+  r = __builtin_fma(r, __builtin_fma(-d, r, 1.0), r);
+  return __builtin_amdgcn_div_fixup(r, d, 1.0);
 }
 
 // Value of the lane before / after / two before within the tile's lanes
@@ -418,55 +480,28 @@ __device__ __forceinline__ double from_prev2_col(double x) {
 }
 
 template <int NL>
-__device__ __forceinline__ Row4 expand_raw(const Raw2 &w, int jj, bool last) {
-  const double m2 = from_prev2_col<NL>(w.c);
+__device__ __forceinline__ Row3 expand_raw(const Raw2 &w, int jj) {
   if constexpr (NL == 16) {
     // a DPP row of 16 lanes is the tile: its first and last lanes, which have
     // no source lane for row_shr:1 / row_shl:1, keep the edge load
-    return Row4{dpp_or<0x111, 0xF>(w.c, w.e), w.c, dpp_or<0x101, 0xF>(w.c, w.e), last ? m2 : 0.0};
+    return Row3{dpp_or<0x111, 0xF>(w.c, w.e), w.c, dpp_or<0x101, 0xF>(w.c, w.e)};
   } else {
     const double l = from_prev_col<NL>(w.c), r = from_next_col<NL>(w.c);
-    return Row4{jj == 0 ? w.e : l, w.c, jj == NL - 1 ? w.e : r, last ? m2 : 0.0};
+    return Row3{jj == 0 ? w.e : l, w.c, jj == NL - 1 ? w.e : r};
   }
 }
+
+// (c A1 f)(i,j) with the scaled entries K of this column over row i of f; on
+// the tile with the grid's last column (ends, the same for every lane) that
+// column adds its j - 2 entry.
 template <int NL>
-__device__ __forceinline__ Row4 expand_raw(const Row4 &w, int, bool) {
-  return w;
-}
-
-// Rows in flight: the edge-and-centre form (neighbours by DPP) or all three
-// columns loaded.
-template <bool NB_DPP>
-struct RawRow {
-  using type = Raw2;
-  static __device__ __forceinline__ Raw2 load(const double *__restrict__ f, unsigned rowoff,
-                                              const LaneCols &lc) {
-    return load_raw2(f, rowoff, lc);
+__device__ __forceinline__ double a1s(const ColOp &K, const Row3 &w, bool ends, bool last) {
+  double v = (K.sup * w.r + K.mid * w.c) + K.sub * w.l;
+  if (ends) {
+    const double m2 = from_prev2_col<NL>(w.c);
+    v = last ? v + K.z * m2 : v;
   }
-  static __device__ __forceinline__ Raw2 load_b(const double *__restrict__ f, unsigned rowb,
-                                                const LaneCols &lc) {
-    return load_raw2_at(f, rowb, lc);
-  }
-  static __device__ __forceinline__ Raw2 zero() { return Raw2{0.0, 0.0}; }
-};
-template <>
-struct RawRow<false> {
-  using type = Row4;
-  static __device__ __forceinline__ Row4 load(const double *__restrict__ f, unsigned rowoff,
-                                              const LaneCols &lc) {
-    return load_row4(f, rowoff, lc);
-  }
-  static __device__ __forceinline__ Row4 load_b(const double *__restrict__ f, unsigned rowb,
-                                                const LaneCols &lc) {
-    return load_row4(f, rowb / 8u, lc);
-  }
-  static __device__ __forceinline__ Row4 zero() { return Row4{0.0, 0.0, 0.0, 0.0}; }
-};
-
-// (c A1 f)(i,j) with the scaled entries K of this column over row i of f (K.z
-// is zero except on the last column).
-__device__ __forceinline__ double a1s(const ColOp &K, const Row4 &w) {
-  return ((K.sup * w.r + K.mid * w.c) + K.sub * w.l) + K.z * w.m2;
+  return v;
 }
 
 // What the sliding window keeps of a row once it has entered: the value at
@@ -479,36 +514,45 @@ struct WinRow {
   double f1u, t1u, f1d, t1y;
 };
 
-template <int MODE>
-__device__ __forceinline__ void enter_row(const VarCol &q, const Row4 &u, const Row4 &y,
-                                          WinRow &w) {
+// (wv . (l, c, r), every operation written out: a rounding that differs here
+// differs in every later step, and the trained surrogates and their gate
+// thresholds follow the labels' last bits.  For the same reason the two rows
+// before a chunk's walk, `first`, keep the order of the fused operations they
+// have always had.)
+__device__ __forceinline__ double row_share(const VarCol &q, const Row3 &w, bool first) {
+  const double t = first ? __builtin_fma(q.wv0, w.l, q.wv1 * w.c) : __builtin_fma(q.wv1, w.c, q.wv0 * w.l);
+  return __builtin_fma(q.wv2, w.r, t);
+}
+
+template <int MODE, int NL, bool HALF, bool FIRST>
+__device__ __forceinline__ void enter_row(const VarCol &q, const Row3 &u, const Row3 &y, bool ends,
+                                          bool last, WinRow &w) {
   constexpr bool HAS_Y = MODE == SM_HV || MODE == SM_CS || MODE == SM_MCS;
   w.uc = u.c;
-  w.urs = q.wv0 * u.l + q.wv1 * u.c + q.wv2 * u.r;
-  if constexpr (MODE != SM_IMPL) w.f1u = a1s(q.f1, u);
-  if constexpr (MODE == SM_FIRST || MODE == SM_CS || MODE == SM_MCS) w.t1u = a1s(q.t1, u);
+  if constexpr (MODE != SM_IMPL) {
+    w.urs = row_share(q, u, FIRST);
+    w.f1u = a1s<NL>(q.f1, u, ends, last);
+  }
+  if constexpr (!HALF && (MODE == SM_FIRST || MODE == SM_CS || MODE == SM_MCS))
+    w.t1u = a1s<NL>(q.t1, u, ends, last);
   if constexpr (HAS_Y) {
-    Row4 d;
-    d.l = y.l - u.l;
-    d.c = y.c - u.c;
-    d.r = y.r - u.r;
-    d.m2 = y.m2 - u.m2;
+    const Row3 d{y.l - u.l, y.c - u.c, y.r - u.r};
     w.dc = d.c;
-    w.drs = q.wv0 * d.l + q.wv1 * d.c + q.wv2 * d.r;
+    w.drs = row_share(q, d, FIRST);
     w.yc = y.c;
-    if constexpr (MODE == SM_HV || MODE == SM_MCS) w.f1d = a1s(q.f1, d);
-    if constexpr (MODE == SM_HV) w.t1y = a1s(q.t1, y);
+    if constexpr (MODE == SM_HV || MODE == SM_MCS) w.f1d = a1s<NL>(q.f1, d, ends, last);
+    if constexpr (MODE == SM_HV) w.t1y = a1s<NL>(HALF ? q.f1 : q.t1, y, ends, last);
   }
 }
 
 // The S = 0 line (row 0 when the spot mesh starts at 0): A1 keeps only the
 // -r/2 of the split, c * (-r/2) * f(i, j).
-template <int MODE>
+template <int MODE, bool HALF>
 __device__ __forceinline__ void zero_line(const VarCol &q, WinRow &w) {
   if constexpr (MODE != SM_IMPL) w.f1u = q.f1.s0 * w.uc;
-  if constexpr (MODE == SM_FIRST || MODE == SM_CS || MODE == SM_MCS) w.t1u = q.t1.s0 * w.uc;
+  if constexpr (!HALF && (MODE == SM_FIRST || MODE == SM_CS || MODE == SM_MCS)) w.t1u = q.t1.s0 * w.uc;
   if constexpr (MODE == SM_HV || MODE == SM_MCS) w.f1d = q.f1.s0 * w.dc;
-  if constexpr (MODE == SM_HV) w.t1y = q.t1.s0 * w.yc;
+  if constexpr (MODE == SM_HV) w.t1y = (HALF ? q.f1.s0 : q.t1.s0) * w.yc;
 }
 
 // Work-group index -> tile index so that consecutive tiles (which share cache
@@ -548,11 +592,10 @@ __device__ __forceinline__ SpotRow quad_row_fields(double2 a, double2 b) {
   return r;
 }
 
-// Wider tiles (8 or 16 columns): the work-group stages the table rows its
-// chunks read into LDS, chunk by chunk (MAXL rows of 12 fields, 2 doubles of
-// padding per chunk so that the chunks of a wave start on different banks),
-// and each lane reads its row with six 16-byte LDS loads (the lanes of a
-// chunk read the same address).
+// Wider tiles (8 to 32 columns): the work-group holds the table rows its chunks
+// read in LDS, chunk by chunk (MAXL rows of 12 fields), and each lane reads
+// its row with six 16-byte LDS loads (the lanes of a chunk read the same
+// address).
 __device__ __forceinline__ SpotRow lds_row_fields(const double *__restrict__ p) {
   const double2 *q = reinterpret_cast<const double2 *>(p);
   const double2 a = q[0], b = q[1], c = q[2], d = q[3], e = q[4], f = q[5];
@@ -565,19 +608,42 @@ __device__ __forceinline__ SpotRow lds_row_fields(const double *__restrict__ p) 
 // unrolled walk and runs out of registers.
 __device__ __forceinline__ void pin(double x) { asm volatile("" ::"v"(x)); }
 
-// A spot sweep: one work-group per (option, NL adjacent variance columns,
-// NL = 4, 8 or 16); thread (jj, ch) = (tid % NL, tid / NL) owns rows
+// A spot sweep: tiles of (option, NL adjacent variance columns), NL = 4, 8, 16
+// or 32; thread (jj, ch) = (tid % NL, tid / NL) owns rows
 // [ch*L, ch*L+L) of column j0+jj through every phase.  The NL lanes of a
 // chunk work on the same rows, so they share the spot-table rows.  Four
 // columns per tile keep a large grid spread over every CU (2048 x 1024: 256
 // tiles); wider tiles make each load of a wave touch fewer, longer row
 // segments, which pays where the batch has tiles to spare.
 //
+// Wide tiles: a work-group takes tile after tile of its XCD's share, and all
+// that a tile waits for is loaded while the tile before it finishes -- its
+// first state rows by the walk's own ring of loads once that tile needs no
+// more rows, its other first values after the walk, its table rows from memory
+// straight into LDS between the scans, its option's record a tile earlier.
+// Before this every tile was a work-group of its own and spent half its life
+// (11,400 of 23,800 cycles on a 256 x 128 grid) on that chain of dependent
+// loads with the CU's other work-group as its only cover.  Neighbouring tiles
+// run side by side on one XCD because each row of a tile also touches the
+// lines of the tiles beside it: walking along an option instead (eight tiles
+// in a row) tripled the bytes fetched and was slower.  On 4,096 such grids the
+// first stage went from 834 to 628 us, the Craig-Sneyd second stage from 1,014
+// to 860 us (one 512-thread work-group per CU on 32 columns); what bounds them
+// now is the memory system: 2.4 and 3.6 GB move at 4.0 to 4.2 TB/s in row
+// segments of 128 to 256 bytes.  Fewer VALU instructions (80 down to 66 per
+// point) or more rows in flight no longer shorten them, and lines touched a
+// tile ahead are evicted from the 4 MB L2 before they are used.
+// Four-column tiles (few tiles, a work-group each) keep the one-tile form.
+//
+// With theta = 1/2 every entry of theta dt A is half the entry of dt A, exactly,
+// so one set of products serves both (HALF): the same bits with 20 fewer
+// registers, which is what lets the Craig-Sneyd stages keep two waves per SIMD
+// without spills.  Other thetas take the general form.
+//
 // The row walk keeps a window of three rows (i-1, i, i+1) of what the stage
 // needs from U and Y2, the loads of rows i+2 and i+3 in flight, and forms the
-// fused right-hand side (and the next stage's explicit term) of row i.  The
-// state rows are loaded with clamped indices; rows past the chunk are
-// computed and discarded.
+// fused right-hand side (and the next stage's explicit term) of row i.  Rows
+// outside the grid read as 0; rows past the chunk are computed and discarded.
 //
 // The LU solve is run in scaled form: with pivots rd = 1/u, multipliers
 // mu_i = -a_i rd_i and n_i = -c_i rd_i, the forward sweep computes
@@ -594,315 +660,475 @@ __device__ __forceinline__ void pin(double x) { asm volatile("" ::"v"(x)); }
 // keeps them out of both chunk maps.  In the last chunk, rows past the grid
 // (i >= nS) have finite values and follow row nS - 1, whose super-diagonal is
 // zero (n = 0), so they do not reach any valid row either way.
-template <int MODE, int THREADS, int NL, int MAXL>
-__global__ void __launch_bounds__(THREADS)
-spot_sweep_kernel(Ctx c, const Tile *__restrict__ tiles, const double *__restrict__ U,
-                  const double *__restrict__ Y, double *__restrict__ out) {
+// An option's record as the lanes of a wave hold it (lane l: its l-th 8-byte
+// word), loaded a tile ahead with a vector load -- a scalar load in flight
+// would make every LDS read of the walk wait for it -- and read out with
+// v_readlane.
+static_assert(sizeof(HOpt) == 17 * 8, "OptWords names HOpt's words");
+struct OptWords {
+  double w;
+  __device__ __forceinline__ void load(const HOpt *o) {
+    const int l = threadIdx.x % 64;
+    w = reinterpret_cast<const double *>(o)[l < 16 ? l : 16];
+  }
+  __device__ __forceinline__ int lo(int k) const {
+    return __builtin_amdgcn_readlane(__double2loint(w), k);
+  }
+  __device__ __forceinline__ double f(int k) const {
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(w), k), lo(k));
+  }
+  __device__ __forceinline__ int64_t i(int k) const {
+    return (int64_t)(((uint64_t)(uint32_t)__builtin_amdgcn_readlane(__double2hiint(w), k) << 32) |
+                     (uint32_t)lo(k));
+  }
+  __device__ __forceinline__ int nS() const { return lo(0); }
+  __device__ __forceinline__ int nv() const { return lo(1); }
+  __device__ __forceinline__ int64_t off() const { return i(2); }
+  __device__ __forceinline__ int64_t so() const { return i(3); }
+  __device__ __forceinline__ int64_t vo() const { return i(4); }
+  __device__ __forceinline__ double r() const { return f(5); }
+  __device__ __forceinline__ double rho_sigma() const { return f(9) * f(8); }
+  __device__ __forceinline__ double dt() const { return f(10); }
+  __device__ __forceinline__ double tdt() const { return f(11); }
+  __device__ __forceinline__ double th() const { return f(12); }
+  __device__ __forceinline__ double Gz() const { return f(15); }
+  __device__ __forceinline__ bool barrier() const { return lo(16) != 0; }
+};
+
+template <int MODE, int THREADS, int NL, int MAXL, bool HALF>
+__device__ __forceinline__ void spot_tiles(const Ctx &c, const Tile *__restrict__ tiles,
+                                           int ntiles, OptWords ow, int start,
+                                           const double *__restrict__ U,
+                                           const double *__restrict__ Y,
+                                           double *__restrict__ out, double *lds) {
   static_assert(NL == 4 || NL == 8 || NL == 16 || NL == 32,
                 "spot tiles are 4, 8, 16 or 32 columns wide");
-  extern __shared__ double lds[];
   constexpr int TPL = THREADS / NL;
   constexpr bool HAS_Y = MODE == SM_HV || MODE == SM_CS || MODE == SM_MCS;
   constexpr bool HAS_EX = MODE != SM_IMPL;
   constexpr bool TAB_LDS = NL != 4;
-  constexpr int CHP = MAXL * kSpFields + 2;  // LDS table: doubles per chunk
+  constexpr bool RUNS = NL != 4;  // several tiles per work-group
+  constexpr int CHP = MAXL * kSpFields;  // LDS table: doubles per chunk
   // state rows in flight (two for the second-stage modes on long chunks,
   // whose window and registers are largest)
-  constexpr int PF = (MODE == SM_HV || MODE == SM_MCS) && MAXL == 16 ? 2 : 4;
-  constexpr bool NB_DPP = true;              // neighbour columns by DPP
-  double *cM = lds;
-  double *cE = cM + NL * (TPL + 1);
-  double *cIn = cE + NL * (TPL + 1);
-  double *eb = cIn + NL * (TPL + 1);  // next stage's explicit term, slot [k * THREADS + tid]
+  constexpr int PF = HAS_Y && MAXL == 16 ? 2 : 4;
+  static_assert(MAXL % PF == 0, "the ring's slots line up from tile to tile");
+  // the chunk carries (four-column tiles: the wave totals of the two scans),
+  // then the next stage's explicit term, slot [k * THREADS + tid], and the
+  // table rows
+  double *cM = lds, *cE = cM + NL * (TPL + 1), *cIn = cE + NL * (TPL + 1);
+  double2 *tot_f = reinterpret_cast<double2 *>(lds), *tot_b = tot_f + THREADS / 64 * 4;
+  double *eb = lds + (NL == 4 ? THREADS / 4 : 3 * NL * (TPL + 1));
   double *tab = eb + (HAS_EX ? MAXL * THREADS : 0);  // 16-byte aligned
-  const Tile t = tiles[xcd_tile(blockIdx.x, gridDim.x)];
-  const HOpt o = c.opts[t.opt];
-  const int nS = (int)o.nS, nv = (int)o.nv, j0 = t.start;
   const int tid = threadIdx.x;
   const int jj = tid % NL, ch = tid / NL;
-  const int j = j0 + jj;
-  const bool col_ok = j < nv;
-  const int jc = col_ok ? j : nv - 1;  // clamped column for loads
-  const int L = (nS + TPL - 1) / TPL;
-  const int s = ch * L;
-  const double *u = U + o.off;
-  const double *y2 = HAS_Y ? Y + o.off : nullptr;
-  const double *rd = c.rd0 + o.off;
-  const double *spr = c.spr + o.so * kSpRow;
-  const unsigned unv = (unsigned)nv;
-  auto clamp_row = [&](int i) { return (unsigned)(i < 0 ? 0 : (i >= nS ? nS - 1 : i)); };
 
-  if constexpr (TAB_LDS) {
-    // table rows of every chunk: TPL * MAXL slots (rows past the grid zero)
+  // A tile's geometry: its option's rows as byte offsets (nS <= 2048 and
+  // nv <= 1024 keep them far below 2^31), this lane's columns and its chunk of
+  // L rows from s on.  The grid's last tile ends on the last column
+  // (build_spot_tiles).
+  struct Geom {
+    unsigned rstep, nbytes;
+    int nS, L, s;
+    LaneCols lc;
+    bool ends;  // the tile holds the grid's last column
+    Buf u, y2;
+  };
+  auto geom_of = [&](const OptWords &w, int j0) {
+    Geom g;
+    const int nv = w.nv();
+    g.nS = w.nS();
+    g.rstep = (unsigned)nv * 8u;
+    g.nbytes = (unsigned)g.nS * g.rstep;
+    g.L = (g.nS + TPL - 1) / TPL;
+    g.s = ch * g.L;
+    const int j = j0 + jj;
+    const int jc = j < nv ? j : nv - 1;  // clamped column for loads
+    const int jm = jc > 0 ? jc - 1 : 0, jp = jc < nv - 1 ? jc + 1 : jc;
+    const int jx = jj == 0 ? jm : (jj == NL - 1 ? jp : jc);
+    g.lc = LaneCols{(unsigned)jc * 8u, (unsigned)jx * 8u, jc == nv - 1, j < nv};
+    g.ends = j0 + NL >= nv;
+    g.u = buf_of(U + w.off(), g.nbytes);
+    g.y2 = buf_of((HAS_Y ? Y : U) + w.off(), g.nbytes);
+    return g;
+  };
+
+  // What a tile needs before its walk starts, loaded while the tile before it
+  // finishes: rows s-1 and s of the window, rows s+1 .. s+PF in flight (row
+  // s+1+m in ring slot m % PF), the pivot of row s-1, the column's variance
+  // coefficients and the option's spot-table rows.
+  Raw2 ru[PF], ry[PF], ua, ub, ya, yb;
+  double rdraw, vtab[7];
+  ya = yb = Raw2{0.0, 0.0};
+  auto load_head = [&](const Geom &g, const OptWords &w) {
+    const unsigned rb = (unsigned)g.s * g.rstep, ra = rb - g.rstep;
+    ua = load_raw2(g.u, ra, g.lc);
+    ub = load_raw2(g.u, rb, g.lc);
+    if constexpr (HAS_Y) {
+      ya = load_raw2(g.y2, ra, g.lc);
+      yb = load_raw2(g.y2, rb, g.lc);
+    }
+    rdraw = buf_load(buf_of(c.rd0 + w.off(), g.nbytes), ra + g.lc.jcb);
+    const char *vt = reinterpret_cast<const char *>(c.vt + w.vo()) + g.lc.jcb;
 #pragma unroll
-    for (int slot = tid; slot < TPL * MAXL; slot += THREADS) {
-      const int cc = slot / MAXL, k = slot % MAXL;
-      const int r = cc * L + k;
-      const double2 *src = reinterpret_cast<const double2 *>(spr + (int64_t)(r < nS ? r : 0) * kSpRow);
-      double2 *dst = reinterpret_cast<double2 *>(tab + cc * CHP + k * kSpFields);
-      const bool in = r < nS;
+    for (int f = 0; f < 7; ++f)
+      vtab[f] = *reinterpret_cast<const double *>(vt + (int64_t)f * c.vt_n * 8);
+  };
+  static_assert(VT_GSUB == 0 && VT_V == 6, "vtab holds the first seven variance fields");
+  // table rows of every chunk, straight from memory into LDS: 16-byte unit e of
+  // the table is fields 2 (e % 6), 2 (e % 6) + 1 of row slot e / 6 (rows past
+  // the grid repeat the last one, whose results are discarded)
+  constexpr int UNITS = TPL * MAXL * kSpFields / 2;
+  static_assert(!TAB_LDS || UNITS % 64 == 0, "whole waves of table units");
+  auto load_table = [&](const Geom &g, const OptWords &w) {
+    const double *spr = c.spr + w.so() * kSpRow;
+    const int wave0 = __builtin_amdgcn_readfirstlane(tid / 64 * 64);
 #pragma unroll
-      for (int part = 0; part < 6; ++part) {
-        const double2 v = src[part];
-        dst[part] = in ? v : make_double2(0.0, 0.0);
+    for (int e0 = 0; e0 < UNITS; e0 += THREADS) {
+      if (UNITS % THREADS == 0 || e0 + wave0 < UNITS) {
+        const int e = e0 + tid, slot = e / 6, part = e % 6;
+        const int r = (slot / MAXL) * g.L + slot % MAXL;
+        load_lds16(spr + (unsigned)((r < g.nS ? r : g.nS - 1) * kSpRow + part * 2),
+                   tab + 2 * (e0 + wave0));
       }
     }
+  };
+  const double *tch = tab + ch * CHP;
+
+  // The work-group's tiles: every `step`-th of its XCD's share of the list
+  // (dispatch places work-group b on XCD b mod 8; tiles next to each other
+  // share cache lines of the state, so they run side by side on one XCD).
+  const int xcd = blockIdx.x % 8, step = ((int)gridDim.x - xcd + 7) / 8;
+  const int share = ntiles / 8 + (xcd < ntiles % 8 ? 1 : 0);
+  const Tile *mine = tiles + xcd * (ntiles / 8) + (xcd < ntiles % 8 ? xcd : ntiles % 8);
+  int at = blockIdx.x / 8;
+  int lane_zero = 0;  // makes the address per-lane, so that the load is a vector load
+  asm volatile("" : "+v"(lane_zero));
+  auto load_tile = [&](int k) { return mine[(k < share ? k : share - 1) + lane_zero]; };
+  // the tile after this one and its option; the one after that
+  Tile t1{0, 0}, t2{0, 0};
+  OptWords on = ow;
+  int start_n = start;
+  if constexpr (RUNS) {
+    t1 = load_tile(at + step);
+    t2 = load_tile(at + 2 * step);
   }
 
-  VarCol q;
-  const bool last = jc == nv - 1;
-  {
-    const double v = VT(c, o, VT_V, jc);
-    q.wv0 = VT(c, o, VT_WSUB, jc); q.wv1 = VT(c, o, VT_WMID, jc); q.wv2 = VT(c, o, VT_WSUP, jc);
-    q.c0h = 0.5 * v;
-    q.rsv = (o.rho * o.sigma) * v;
-    const double gsub = VT(c, o, VT_GSUB, jc), gmid = VT(c, o, VT_GMID, jc),
-                 gsup = VT(c, o, VT_GSUP, jc), gz = last ? o.Gz : 0.0, split = -o.r / 2.0;
-    q.f1 = col_op(o.dt, gsub, gmid, gsup, gz, split);
-    q.t1 = col_op(o.tdt, gsub, gmid, gsup, gz, split);
-  }
-  LaneCols lc;
-  lc.jc = (unsigned)jc;
-  lc.jm = jc > 0 ? lc.jc - 1 : 0u;
-  lc.jp = jc < nv - 1 ? lc.jc + 1 : lc.jc;
-  lc.jm2 = jc > 1 ? lc.jc - 2 : 0u;
-  lc.jx = jj == 0 ? lc.jm : (jj == NL - 1 ? lc.jp : lc.jc);
-  lc.last = last;
-  const double tdt = o.tdt, dt = o.dt;
-  const bool barrier = o.barrier != 0;
-  // S = 0 line (row 0 when the mesh starts at 0): A1 keeps only the -r/2 split
-  const bool s0_zero = s == 0 && spr[13] == 0.0;
-
-  // Pivot recurrence state from the row before the chunk.
-  double rdp = 0.0, cp = 0.0;
-  if (s > 0) {
-    const double *pr = spr + (int64_t)(s - 1) * kSpRow;
-    const double c00 = q.c0h * pr[11];
-    rdp = rd[(unsigned)(s - 1) * unv + lc.jc];
-    cp = -tdt * band_add(pr[2], pr[5], c00);
-  }
-
-  // Window: rows s-1 (a) and s (b) entered; rows s+1 .. s+PF in flight
-  // (row s+1+m in ring slot m % PF).
-  WinRow wa, wb, wc;
-  {
-    const Row4 z{0.0, 0.0, 0.0, 0.0};
-    const Row4 ua = load_row4(u, clamp_row(s - 1) * unv, lc);
-    const Row4 ub = load_row4(u, clamp_row(s) * unv, lc);
-    Row4 ya = z, yb = z;
-    if constexpr (HAS_Y) {
-      ya = load_row4(y2, clamp_row(s - 1) * unv, lc);
-      yb = load_row4(y2, clamp_row(s) * unv, lc);
-    }
-    enter_row<MODE>(q, ua, ya, wa);
-    enter_row<MODE>(q, ub, yb, wb);
-    if (s0_zero) zero_line<MODE>(q, wb);
-  }
-  using RR = RawRow<NB_DPP>;
-  typename RR::type ru[PF], ry[PF];
+  Geom g = geom_of(ow, start);
+  if constexpr (TAB_LDS) load_table(g, ow);
+  load_head(g, ow);
 #pragma unroll
   for (int m = 0; m < PF; ++m) {
-    const unsigned rr = clamp_row(s + 1 + m) * unv;
-    ru[m] = RR::load(u, rr, lc);
-    ry[m] = RR::zero();
-    if constexpr (HAS_Y) ry[m] = RR::load(y2, rr, lc);
+    const unsigned rr = (unsigned)(g.s + 1 + m) * g.rstep;
+    ru[m] = load_raw2(g.u, rr, g.lc);
+    ry[m] = Raw2{0.0, 0.0};
+    if constexpr (HAS_Y) ry[m] = load_raw2(g.y2, rr, g.lc);
   }
-  // four-column tiles: table rows i and i+1 in flight
-  double2 ta0, tb0, ta1, tb1;
-  if constexpr (!TAB_LDS) {
-    quad_row_load(spr + clamp_row(s) * kSpRow, jj, ta0, tb0);
-    quad_row_load(spr + clamp_row(s + 1) * kSpRow, jj, ta1, tb1);
+  if constexpr (RUNS) {
+    on.load(c.opts + __builtin_amdgcn_readfirstlane(t1.opt));
+    start_n = __builtin_amdgcn_readfirstlane(t1.start);
   }
-  if constexpr (TAB_LDS) __syncthreads();
-  const double *tch = tab + ch * CHP;
-  // byte offset of the row the walk loads next (row s + 1 + PF + k at step k),
-  // clamped to the last row; nS <= 2048 and nv <= 1024 keep it far below 2^32
-  const unsigned rstep = unv * 8u, rlast = (unsigned)(nS - 1) * rstep;
-  unsigned rnext = (unsigned)(s + 1 + PF) * rstep;
+  if constexpr (TAB_LDS) {
+    lds_loads_done();
+    __syncthreads();
+  }
 
-  double mu[MAXL], nreg[MAXL], dv[MAXL];
-#pragma unroll
-  for (int k = 0; k < MAXL; ++k) {
-    const int i = s + k;
-    const int slot = k % PF;
-    // the table row of row i
-    SpotRow R;
-    double2 ta2, tb2;
-    if constexpr (TAB_LDS) {
-      R = lds_row_fields(tch + k * kSpFields);
-    } else {
-      quad_row_load(spr + clamp_row(i + 2) * kSpRow, jj, ta2, tb2);
-    }
-    // row i + 1 enters the window; its slot takes the loads of row i + 1 + PF
+  for (;;) {
+    const bool more = RUNS && at + step < share;
+    const int nS = g.nS, L = g.L, s = g.s;
+    const unsigned rstep = g.rstep;
+    const LaneCols lc = g.lc;
+    const Buf u = g.u, y2 = g.y2;
+    const double tdt = ow.tdt(), dt = ow.dt();
+    const double *spr = c.spr + ow.so() * kSpRow;
+    auto clamp_row = [&](int i) { return (unsigned)(i < 0 ? 0 : (i >= nS ? nS - 1 : i)); };
+    VarCol q;
     {
-      const Row4 un = expand_raw<NL>(ru[slot], jj, last);
-      Row4 yn{0.0, 0.0, 0.0, 0.0};
-      if constexpr (HAS_Y) yn = expand_raw<NL>(ry[slot], jj, last);
-      enter_row<MODE>(q, un, yn, wc);
-      const unsigned rb = rnext < rlast ? rnext : rlast;
-      rnext += rstep;
-      ru[slot] = RR::load_b(u, rb, lc);
-      if constexpr (HAS_Y) ry[slot] = RR::load_b(y2, rb, lc);
+      q.wv0 = vtab[VT_WSUB]; q.wv1 = vtab[VT_WMID]; q.wv2 = vtab[VT_WSUP];
+      q.c0h = 0.5 * vtab[VT_V];
+      q.rsv = ow.rho_sigma() * vtab[VT_V];
+      const double gz = lc.last ? ow.Gz() : 0.0, split = -ow.r() / 2.0;
+      q.f1 = col_op(dt, vtab[VT_GSUB], vtab[VT_GMID], vtab[VT_GSUP], gz, split);
+      if constexpr (!HALF)
+        q.t1 = col_op(tdt, vtab[VT_GSUB], vtab[VT_GMID], vtab[VT_GSUP], gz, split);
     }
-    if constexpr (!TAB_LDS) R = quad_row_fields(ta0, tb0);
-
-    const Bands B = a0_bands(R, q.c0h);
-    // the entries of dt A0 and theta dt A0, fl(c * a), as the reference's
-    // scaled operators hold them; applied in its band order (super, main, sub)
-    const double tsub = tdt * B.sub, tmid = tdt * B.mid, tsup = tdt * B.sup;
-    double rhs = 0.0, ex = 0.0;
-    if constexpr (MODE == SM_IMPL) {
-      rhs = wb.uc + dt * B.r0;
-    } else {
-      const double dsub = dt * B.sub, dmid = dt * B.mid, dsup = dt * B.sup;
-      auto a0d = [&](double xa, double xb, double xc) {
-        return (dsup * xc + dmid * xb) + dsub * xa;
-      };
-      auto a0t = [&](double xa, double xb, double xc) {
-        return (tsup * xc + tmid * xb) + tsub * xa;
-      };
-      // (A01 f)(i, j) from the rows' shares
-      auto x01 = [&](double ra, double rb, double rc) {
-        return q.rsv * (R.wsub * ra + R.wmid * rb + R.wsup * rc);
-      };
-      // Y0 = U + dt A0 U + dt R0 + dt A01 U + dt A1 U, in the reference's
-      // order of its explicit operators (spot, cross, variance)
-      const double y0 = ((wb.uc + (a0d(wa.uc, wb.uc, wc.uc) + dt * B.r0)) +
-                         dt * x01(wa.urs, wb.urs, wc.urs)) +
-                        wb.f1u;
-      if constexpr (MODE == SM_FIRST) {
-        rhs = y0 - a0t(wa.uc, wb.uc, wc.uc);
-        ex = wb.t1u;
-      } else if constexpr (MODE == SM_HV) {
-        // the second-stage corrections act on the difference of the states
-        // (FiniteDifferenceEngine.pyx:744-765, 818-835, 881-894)
-        // V = Y0 - 1/2 F (U - Y2) over the explicit operators (no residual)
-        const double v1 = ((y0 + 0.5 * a0d(wa.dc, wb.dc, wc.dc)) +
-                           0.5 * (dt * x01(wa.drs, wb.drs, wc.drs))) +
-                          0.5 * wb.f1d;
-        rhs = v1 - a0t(wa.yc, wb.yc, wc.yc);
-        ex = wb.t1y;
-      } else if constexpr (MODE == SM_CS) {
-        rhs = (y0 + (0.5 * dt) * x01(wa.drs, wb.drs, wc.drs)) - a0t(wa.uc, wb.uc, wc.uc);
-        ex = wb.t1u;
-      } else {  // SM_MCS: (1/2 - theta) F (Y2 - U), residual included
-        const double h = 0.5 - o.th;
-        const double xd = x01(wa.drs, wb.drs, wc.drs);
-        const double v1 = (((y0 + tdt * xd) + h * (a0d(wa.dc, wb.dc, wc.dc) + dt * B.r0)) +
-                           h * (dt * xd)) +
-                          h * wb.f1d;
-        rhs = v1 - a0t(wa.uc, wb.uc, wc.uc);
-        ex = wb.t1u;
-      }
-    }
-    // the solve forces Dirichlet rows (0, and nS-1 under a barrier) to 0
-    if ((k == 0 && s == 0) || (barrier && i == nS - 1)) rhs = 0.0;
-    // I - tdt*A0 on this row (identity rows on Dirichlet rows and zero
-    // off-diagonals at the line ends come from the bands), scaled by the
-    // pivot.  The diagonal 1 - tdt*b is one fused operation, as the
-    // factorisation forms it (li0_row), written out so that the compiler's
-    // contraction choices cannot change how the recomputed pivots round.
-    const double rd0 = 1.0 / (__builtin_fma(-tdt, B.mid, 1.0) - (-tsub * rdp) * cp);
-    rdp = rd0;
-    cp = -tsup;
-    const double dsc = rd0 * rhs;
-    mu[k] = tsub * rd0;
-    nreg[k] = tsup * rd0;
-    dv[k] = dsc;
-    if constexpr (HAS_EX) eb[k * THREADS + tid] = ex;
-    // slide the window
-    wa = wb;
-    wb = wc;
+    // four-column tiles: table rows i and i+1 in flight
+    double2 ta0, tb0, ta1, tb1;
     if constexpr (!TAB_LDS) {
-      ta0 = ta1; tb0 = tb1; ta1 = ta2; tb1 = tb2;
+      quad_row_load(spr + clamp_row(s) * kSpRow, jj, ta0, tb0);
+      quad_row_load(spr + clamp_row(s + 1) * kSpRow, jj, ta1, tb1);
     }
-    // this row's results before the next row's loads (registers)
-    pin(dsc);
-    pin(rdp);
-    if constexpr (HAS_EX) pin(ex);
-    __builtin_amdgcn_sched_barrier(0);
-  }
-  // Chunk maps and fix-ups.  Rows k >= L belong to the next chunk; L is
-  // uniform, so full chunks (L == MAXL, the common case) take unguarded loops.
-  const bool full = L == MAXL;
-  const bool active = col_ok && s < nS;
-  double M = 1.0, E = 0.0;
-  if (full) {
+    // Pivot recurrence state from the row before the chunk.
+    double rdp = 0.0, cp = 0.0;
+    if (s > 0) {
+      const double *pr =
+          TAB_LDS ? tch - CHP + (L - 1) * kSpFields : spr + clamp_row(s - 1) * kSpRow;
+      const double c00 = q.c0h * pr[11];
+      rdp = rdraw;
+      cp = -tdt * band_add(pr[2], pr[5], c00);
+    }
+    WinRow wa, wb, wc;
+    const bool ends = g.ends;
+    enter_row<MODE, NL, HALF, true>(q, expand_raw<NL>(ua, jj), expand_raw<NL>(ya, jj), ends, lc.last, wa);
+    enter_row<MODE, NL, HALF, true>(q, expand_raw<NL>(ub, jj), expand_raw<NL>(yb, jj), ends, lc.last, wb);
+    // the S = 0 line (row 0 when the mesh starts at 0): A1 keeps only the -r/2
+    // of the split
+    if (s == 0 && (TAB_LDS ? tch[11] : spr[11]) == 0.0) zero_line<MODE, HALF>(q, wb);
+    // the next tile (this one again after the last)
+    const Geom gn = RUNS ? geom_of(on, start_n) : g;
+    // byte offsets of the row the walk loads next (row s + 1 + PF + k at step
+    // k), at the column and at the edge column
+    unsigned oc = (unsigned)(s + 1 + PF) * rstep + lc.jcb, ox = oc - lc.jcb + lc.jxb;
+
+    double mu[MAXL], nreg[MAXL], dv[MAXL];
 #pragma unroll
     for (int k = 0; k < MAXL; ++k) {
-      E = dv[k] + mu[k] * E;
-      M = mu[k] * M;
+      const int slot = k % PF;
+      // the table row of row s + k
+      SpotRow R;
+      double2 ta2, tb2;
+      if constexpr (TAB_LDS) {
+        R = lds_row_fields(tch + k * kSpFields);
+      } else {
+        quad_row_load(spr + clamp_row(s + k + 2) * kSpRow, jj, ta2, tb2);
+      }
+      // row s + k + 1 enters the window; its slot takes the loads of row
+      // s + k + 1 + PF, or, where this tile needs no more rows, the next
+      // tile's row of that slot
+      {
+        const Row3 un = expand_raw<NL>(ru[slot], jj);
+        Row3 yn{0.0, 0.0, 0.0};
+        if constexpr (HAS_Y) yn = expand_raw<NL>(ry[slot], jj);
+        enter_row<MODE, NL, HALF, false>(q, un, yn, ends, lc.last, wc);
+        if (RUNS && k == MAXL - PF) {
+          oc = (unsigned)(gn.s + 1) * gn.rstep + gn.lc.jcb;
+          ox = oc - gn.lc.jcb + gn.lc.jxb;
+        }
+        const bool here = k < MAXL - PF;
+        if (RUNS || here) {
+          const Buf bu = here ? u : gn.u, by = here ? y2 : gn.y2;
+          ru[slot] = Raw2{buf_load(bu, ox), buf_load(bu, oc)};
+          if constexpr (HAS_Y) ry[slot] = Raw2{buf_load(by, ox), buf_load(by, oc)};
+        }
+        oc += here ? rstep : gn.rstep;
+        ox += here ? rstep : gn.rstep;
+      }
+      if constexpr (!TAB_LDS) R = quad_row_fields(ta0, tb0);
+
+      const Bands B = a0_bands(R, q.c0h);
+      // the entries of dt A0 and theta dt A0, fl(c * a), as the reference's
+      // scaled operators hold them; applied in its band order (super, main,
+      // sub).  With theta = 1/2 the latter are half the former, exactly, and so
+      // is every product and sum of them.
+      const double dsub = dt * B.sub, dmid = dt * B.mid, dsup = dt * B.sup;
+      const double tsub = HALF ? 0.5 * dsub : tdt * B.sub, tsup = HALF ? 0.5 * dsup : tdt * B.sup;
+      const double tmid = tdt * B.mid;
+      double rhs = 0.0, ex = 0.0;
+      if constexpr (MODE == SM_IMPL) {
+        rhs = wb.uc + dt * B.r0;
+      } else {
+        auto a0d = [&](double xa, double xb, double xc) {
+          return (dsup * xc + dmid * xb) + dsub * xa;
+        };
+        // d - (theta dt A0 x), given a = dt A0 x
+        auto less_a0t = [&](double d, double a, double xa, double xb, double xc) {
+          if constexpr (HALF) return __builtin_fma(-0.5, a, d);
+          return d - ((tsup * xc + tmid * xb) + tsub * xa);
+        };
+        // (A01 f)(i, j) from the rows' shares
+        auto x01 = [&](double ra, double rb, double rc) {
+          return q.rsv * (R.wsub * ra + R.wmid * rb + R.wsup * rc);
+        };
+        // Y0 = U + dt A0 U + dt R0 + dt A01 U + dt A1 U, in the reference's
+        // order of its explicit operators (spot, cross, variance)
+        const double a0 = a0d(wa.uc, wb.uc, wc.uc);
+        const double y0 =
+            ((wb.uc + (a0 + dt * B.r0)) + dt * x01(wa.urs, wb.urs, wc.urs)) + wb.f1u;
+        ex = HALF ? wb.f1u : wb.t1u;
+        if constexpr (MODE == SM_FIRST) {
+          rhs = less_a0t(y0, a0, wa.uc, wb.uc, wc.uc);
+        } else if constexpr (MODE == SM_HV) {
+          // the second-stage corrections act on the difference of the states
+          // (FiniteDifferenceEngine.pyx:744-765, 818-835, 881-894)
+          // V = Y0 - 1/2 F (U - Y2) over the explicit operators (no residual)
+          const double v1 = ((y0 + 0.5 * a0d(wa.dc, wb.dc, wc.dc)) +
+                             0.5 * (dt * x01(wa.drs, wb.drs, wc.drs))) +
+                            0.5 * wb.f1d;
+          rhs = less_a0t(v1, HALF ? a0d(wa.yc, wb.yc, wc.yc) : 0.0, wa.yc, wb.yc, wc.yc);
+          ex = wb.t1y;
+        } else if constexpr (MODE == SM_CS) {
+          rhs = less_a0t(y0 + (0.5 * dt) * x01(wa.drs, wb.drs, wc.drs), a0, wa.uc, wb.uc, wc.uc);
+        } else {  // SM_MCS: (1/2 - theta) F (Y2 - U), residual included
+          const double h = 0.5 - ow.th();
+          const double xd = x01(wa.drs, wb.drs, wc.drs);
+          const double v1 = (((y0 + tdt * xd) + h * (a0d(wa.dc, wb.dc, wc.dc) + dt * B.r0)) +
+                             h * (dt * xd)) +
+                            h * wb.f1d;
+          rhs = less_a0t(v1, a0, wa.uc, wb.uc, wc.uc);
+        }
+      }
+      // the solve forces the Dirichlet row 0 to 0 (a barrier's row below)
+      if (k == 0 && s == 0) rhs = 0.0;
+      // I - tdt*A0 on this row (identity rows on Dirichlet rows and zero
+      // off-diagonals at the line ends come from the bands), scaled by the
+      // pivot.  The diagonal 1 - tdt*b is one fused operation, as the
+      // factorisation forms it (li0_row), written out so that the compiler's
+      // contraction choices cannot change how the recomputed pivots round.
+      const double rd0 = recip(__builtin_fma(-tdt, B.mid, 1.0) - (-tsub * rdp) * cp);
+      rdp = rd0;
+      cp = -tsup;
+      const double dsc = rd0 * rhs;
+      mu[k] = tsub * rd0;
+      nreg[k] = tsup * rd0;
+      dv[k] = dsc;
+      if constexpr (HAS_EX) eb[k * THREADS + tid] = ex;
+      // slide the window
+      wa = wb;
+      wb = wc;
+      if constexpr (!TAB_LDS) {
+        ta0 = ta1; tb0 = tb1; ta1 = ta2; tb1 = tb2;
+      }
+      // this row's results before the next row's loads (registers)
+      pin(dsc);
+      pin(rdp);
+      if constexpr (HAS_EX) pin(ex);
+      __builtin_amdgcn_sched_barrier(0);
     }
-  } else {
+    // (also after the last tile, which is then loaded again: a branch would
+    // keep this tile's values alive through the walk)
+    const bool barrier = ow.barrier();
+    const Buf ob = buf_of(out + ow.off(), g.nbytes);
+    if constexpr (RUNS) {
+      load_head(gn, on);
+    }
+    // a barrier's Dirichlet row (its bands are zero, its pivot 1)
+    if (barrier) {
 #pragma unroll
-    for (int k = 0; k < MAXL; ++k) {
-      if (k < L) {
+      for (int k = 0; k < MAXL; ++k)
+        if (s + k == nS - 1) dv[k] = 0.0;
+    }
+    // Chunk maps and fix-ups.  Rows k >= L belong to the next chunk; L is
+    // uniform, so full chunks (L == MAXL, the common case) take unguarded loops.
+    const bool full = L == MAXL;
+    const bool active = lc.ok && s < nS;
+    double M = 1.0, E = 0.0;
+    if (full) {
+#pragma unroll
+      for (int k = 0; k < MAXL; ++k) {
         E = dv[k] + mu[k] * E;
         M = mu[k] * M;
       }
+    } else {
+#pragma unroll
+      for (int k = 0; k < MAXL; ++k) {
+        if (k < L) {
+          E = dv[k] + mu[k] * E;
+          M = mu[k] * M;
+        }
+      }
     }
-  }
-  cM[jj * (TPL + 1) + ch] = active ? M : 1.0;
-  cE[jj * (TPL + 1) + ch] = active ? E : 0.0;
-  __syncthreads();
-  affine_scan<THREADS, NL, false>(cM, cE, cIn);
-  __syncthreads();
-  // Forward fix-up, then the local backward recurrence x = y' + n x'.
-  {
-    double yv = cIn[jj * (TPL + 1) + ch];
+    double yv = 0.0;
+    if constexpr (NL == 4) {
+      yv = quad_carry<THREADS, false>(active ? M : 1.0, active ? E : 0.0, tot_f);
+    } else {
+      cM[jj * (TPL + 1) + ch] = active ? M : 1.0;
+      cE[jj * (TPL + 1) + ch] = active ? E : 0.0;
+      __syncthreads();
+      // every wave is past its walk
+      // the next tile's table rows, and the records of the tiles after it
+      load_table(gn, on);
+      ow = on;
+      on.load(c.opts + __builtin_amdgcn_readfirstlane(t2.opt));
+      start_n = __builtin_amdgcn_readfirstlane(t2.start);
+      t2 = load_tile(at + 3 * step);
+      affine_scan<THREADS, NL, false>(cM, cE, cIn);
+      __syncthreads();
+      yv = cIn[jj * (TPL + 1) + ch];
+    }
+    // Forward fix-up, then the local backward recurrence x = y' + n x'.
 #pragma unroll
     for (int k = 0; k < MAXL; ++k) {
       yv = dv[k] + mu[k] * yv;
       dv[k] = yv;
     }
-  }
-  M = 1.0;
-  E = 0.0;
-  if (full) {
+    M = 1.0;
+    E = 0.0;
+    if (full) {
 #pragma unroll
-    for (int k = MAXL - 1; k >= 0; --k) {
-      E = dv[k] + nreg[k] * E;
-      M = nreg[k] * M;
-    }
-  } else {
-#pragma unroll
-    for (int k = MAXL - 1; k >= 0; --k) {
-      if (k < L) {
+      for (int k = MAXL - 1; k >= 0; --k) {
         E = dv[k] + nreg[k] * E;
         M = nreg[k] * M;
       }
-    }
-  }
-  __syncthreads();  // everyone done reading cIn of the forward scan
-  cM[jj * (TPL + 1) + ch] = active ? M : 1.0;
-  cE[jj * (TPL + 1) + ch] = active ? E : 0.0;
-  __syncthreads();
-  affine_scan<THREADS, NL, true>(cM, cE, cIn);
-  __syncthreads();
-  // Backward fix-up; stage output x - tdt*A1(f) written straight from the chunk.
-  double *ob = out + o.off;
-  double x = cIn[jj * (TPL + 1) + ch];
-  // byte offset of (row s + k, column j), stepped down the chunk
-  unsigned sb = (unsigned)(s + MAXL - 1) * rstep + (unsigned)j * 8u;
-  if (full) {
+    } else {
 #pragma unroll
-    for (int k = MAXL - 1; k >= 0; --k) {
-      const int i = s + k;
-      x = dv[k] + nreg[k] * x;
-      if (col_ok && i < nS) store_at(ob, sb, HAS_EX ? x - eb[k * THREADS + tid] : x);
-      sb -= rstep;
-    }
-  } else {
-#pragma unroll
-    for (int k = MAXL - 1; k >= 0; --k) {
-      const int i = s + k;
-      if (k < L) {
-        x = dv[k] + nreg[k] * x;
-        if (col_ok && i < nS) store_at(ob, sb, HAS_EX ? x - eb[k * THREADS + tid] : x);
+      for (int k = MAXL - 1; k >= 0; --k) {
+        if (k < L) {
+          E = dv[k] + nreg[k] * E;
+          M = nreg[k] * M;
+        }
       }
-      sb -= rstep;
     }
+    double x = 0.0;
+    if constexpr (NL == 4) {
+      x = quad_carry<THREADS, true>(active ? M : 1.0, active ? E : 0.0, tot_b);
+    } else {
+      __syncthreads();  // everyone done reading cIn of the forward scan
+      cM[jj * (TPL + 1) + ch] = active ? M : 1.0;
+      cE[jj * (TPL + 1) + ch] = active ? E : 0.0;
+      __syncthreads();
+      affine_scan<THREADS, NL, true>(cM, cE, cIn);
+      lds_loads_done();
+      __syncthreads();  // the carries, and the next tile's table rows
+      x = cIn[jj * (TPL + 1) + ch];
+    }
+    // Backward fix-up; stage output x - tdt*A1(f) written straight from the
+    // chunk (rows past the grid and lanes past its columns fall outside the
+    // buffer).
+    // byte offset of (row s + k, column j), stepped down the chunk
+    unsigned sb = lc.ok ? (unsigned)(s + MAXL - 1) * rstep + lc.jcb : 0xfffffff8u;
+    auto put = [&](int k) {
+      double v = x;
+      if constexpr (HAS_EX) {
+        const double ex = eb[k * THREADS + tid];
+        v = HALF ? __builtin_fma(-0.5, ex, x) : x - ex;
+      }
+      buf_store(ob, sb, v);
+    };
+    if (full) {
+#pragma unroll
+      for (int k = MAXL - 1; k >= 0; --k) {
+        x = dv[k] + nreg[k] * x;
+        put(k);
+        sb -= rstep;
+      }
+    } else {
+#pragma unroll
+      for (int k = MAXL - 1; k >= 0; --k) {
+        if (k < L) {
+          x = dv[k] + nreg[k] * x;
+          put(k);
+        }
+        sb -= rstep;
+      }
+    }
+    if (!more) break;
+    at += step;
+    g = gn;
   }
+}
+
+template <int MODE, int THREADS, int NL, int MAXL>
+__global__ void __launch_bounds__(THREADS, THREADS == 256 ? 2 : 1)
+spot_sweep_kernel(Ctx c, const Tile *__restrict__ tiles, int ntiles, const double *__restrict__ U,
+                  const double *__restrict__ Y, double *__restrict__ out) {
+  extern __shared__ double lds[];
+  const Tile t = tiles[xcd_tile(blockIdx.x, ntiles)];
+  OptWords o;
+  o.load(c.opts + t.opt);
+  if (MODE != SM_IMPL && o.th() == 0.5)
+    spot_tiles<MODE, THREADS, NL, MAXL, MODE != SM_IMPL>(c, tiles, ntiles, o, t.start, U, Y, out, lds);
+  else
+    spot_tiles<MODE, THREADS, NL, MAXL, false>(c, tiles, ntiles, o, t.start, U, Y, out, lds);
 }
 
 // ---- variance sweep -------------------------------------------------------------
@@ -1501,27 +1727,28 @@ int spot_group_of(const std::vector<std::pair<int, int>> &c, int nl, int64_t nS)
 int build_spot_tiles(fdadi_hb *hb) {
   std::vector<Tile> st;
   hb->sgroups.clear();
-  auto add_tiles = [&](int k) {
-    const HOpt &o = hb->h_opts[k];
-    // the last tile ends on the last column (it may overlap the one before,
-    // whose shared columns both compute identically): the kernel takes
-    // column nv - 3 of the last column from the lane two before it
-    for (int64_t j0 = 0; j0 < o.nv; j0 += hb->spot_nl) {
-      const int64_t start = j0 + hb->spot_nl > o.nv && o.nv >= hb->spot_nl ? o.nv - hb->spot_nl : j0;
-      st.push_back(Tile{k, (int32_t)start});
+  const int nl = hb->spot_nl;
+  auto add_group = [&](int threads, int maxl, const std::vector<int> &opts) {
+    const int first = (int)st.size();
+    for (int k : opts) {
+      const HOpt &o = hb->h_opts[k];
+      // the last tile ends on the last column (it may overlap the one before,
+      // whose shared columns both compute identically): the kernel takes
+      // column nv - 3 of the last column from the lane two before it
+      for (int64_t j0 = 0; j0 < o.nv; j0 += nl)
+        st.push_back(Tile{k, (int32_t)(j0 + nl > o.nv && o.nv >= nl ? o.nv - nl : j0)});
     }
+    hb->sgroups.push_back({threads, maxl, first, (int)st.size() - first});
   };
   if (!hb->spot_split) {
-    for (int k : hb->order) add_tiles(k);
-    hb->sgroups.push_back({hb->spot_threads, hb->spot_maxl, 0, (int)st.size()});
+    add_group(hb->spot_threads, hb->spot_maxl, hb->order);
   } else {
-    const auto c = spot_candidates(hb->spot_nl);
+    const auto c = spot_candidates(nl);
     for (size_t g = 0; g < c.size(); ++g) {
-      const int first = (int)st.size();
+      std::vector<int> opts;
       for (int k : hb->order)  // largest first within a group
-        if (spot_group_of(c, hb->spot_nl, hb->h_opts[k].nS) == (int)g) add_tiles(k);
-      if ((int)st.size() > first)
-        hb->sgroups.push_back({c[g].first, c[g].second, first, (int)st.size() - first});
+        if (spot_group_of(c, nl, hb->h_opts[k].nS) == (int)g) opts.push_back(k);
+      if (!opts.empty()) add_group(c[g].first, c[g].second, opts);
     }
   }
   FDADI_REQUIRE((int64_t)st.size() <= hb->cap_stiles, FDADI_ERR_STATE,
@@ -1590,14 +1817,17 @@ int launch_spot_t(const fdadi_hb *hb, const fdadi_hb::SweepGroup &g, const doubl
                   const double *Y, double *out, hipStream_t s) {
   constexpr int TPL = T / NL;
   // chunk carries of the scans, the next stage's explicit term (MAXL per
-  // thread); wide tiles add their table rows (MAXL rows of 12 fields + 2
-  // doubles of padding per chunk)
+  // thread); wide tiles add their table rows (MAXL rows of 12 fields per chunk)
   const size_t ex = MODE == SM_IMPL ? 0 : (size_t)ML * T;
-  const size_t tab = NL == 4 ? 0 : (size_t)TPL * (ML * 12 + 2);
-  const size_t lds = sizeof(double) * (3 * (size_t)NL * (TPL + 1) + ex + tab);
+  const size_t tab = NL == 4 ? 0 : (size_t)TPL * ML * kSpFields;
+  const size_t carry = NL == 4 ? T / 4 : 3 * (size_t)NL * (TPL + 1);
+  const size_t lds = sizeof(double) * (carry + ex + tab);
   FDADI_RET(allow_lds((const void *)spot_sweep_kernel<MODE, T, NL, ML>, lds));
-  hipLaunchKernelGGL((spot_sweep_kernel<MODE, T, NL, ML>), dim3(g.ntiles), dim3(T), lds, s,
-                     ctx_of(hb), hb->d_stiles + g.first, U, Y, out);
+  // wide tiles: as many work-groups as run at once (two of 256 threads or one
+  // of 512 per CU), each taking tile after tile
+  const int slots = NL == 4 ? g.ntiles : 256 * 512 / T;
+  hipLaunchKernelGGL((spot_sweep_kernel<MODE, T, NL, ML>), dim3(std::min(g.ntiles, slots)),
+                     dim3(T), lds, s, ctx_of(hb), hb->d_stiles + g.first, g.ntiles, U, Y, out);
   FDADI_CHECK_LAUNCH();
   return FDADI_OK;
 }
