@@ -38,7 +38,7 @@ namespace {
 
 enum SpotField {
   SP_PSUB, SP_PMID, SP_PSUP, SP_QSUB, SP_QMID, SP_QSUP, SP_PR, SP_QR,
-  SP_WSUB, SP_WMID, SP_WSUP, SP_S, SP_DIR, SP_NF
+  SP_WSUB, SP_WMID, SP_WSUP, SP_S, SP_NF
 };
 enum VarField {
   VT_GSUB, VT_GMID, VT_GSUP, VT_WSUB, VT_WMID, VT_WSUP, VT_V, VT_M, VT_RD, VT_N, VT_NF
@@ -118,21 +118,6 @@ __device__ double a01_dot(const Ctx &c, const HOpt &o, int64_t i, int64_t j, F x
   }
   const double coef = ((o.rho * o.sigma) * SP(c, o, SP_S, i)) * VT(c, o, VT_V, j);
   return coef * acc;
-}
-
-// Coefficients of the tridiagonal I - tdt*A0 on spot line j at row i.
-__device__ __forceinline__ void li0_row(const Ctx &c, const HOpt &o, int64_t i, double v,
-                                        double &a, double &b, double &cc) {
-  if (SP(c, o, SP_DIR, i) != 0.0) {
-    a = 0.0; b = 1.0; cc = 0.0;
-    return;
-  }
-  const double c00 = c00_of(v, SP(c, o, SP_S, i));
-  a = -o.tdt * band_add(SP(c, o, SP_PSUB, i), SP(c, o, SP_QSUB, i), c00);
-  b = 1.0 - o.tdt * band_add(SP(c, o, SP_PMID, i), SP(c, o, SP_QMID, i), c00);
-  cc = -o.tdt * band_add(SP(c, o, SP_PSUP, i), SP(c, o, SP_QSUP, i), c00);
-  if (i == 0) a = 0.0;
-  if (i == o.nS - 1) cc = 0.0;
 }
 
 // ---- wave-level scans of affine maps ------------------------------------------
@@ -971,8 +956,8 @@ __device__ __forceinline__ void spot_tiles(const Ctx &c, const Tile *__restrict_
       if (k == 0 && s == 0) rhs = 0.0;
       // I - tdt*A0 on this row (identity rows on Dirichlet rows and zero
       // off-diagonals at the line ends come from the bands), scaled by the
-      // pivot.  The diagonal 1 - tdt*b is one fused operation, as the
-      // factorisation forms it (li0_row), written out so that the compiler's
+      // pivot.  The diagonal 1 - tdt*b is one fused operation, as
+      // spot_factor_kernel forms it, written out so that the compiler's
       // contraction choices cannot change how the recomputed pivots round.
       const double rd0 = recip(__builtin_fma(-tdt, B.mid, 1.0) - (-tsub * rdp) * cp);
       rdp = rd0;
@@ -1342,7 +1327,6 @@ __global__ void spot_tables_kernel(const HOpt *opts, int nopt, const int64_t *ro
   col[SP_WMID * sp_n] = ws[1];
   col[SP_WSUP * sp_n] = ws[2];
   col[SP_S * sp_n] = S;
-  col[SP_DIR * sp_n] = dir ? 1.0 : 0.0;
   // AoS row of the spot sweep (layout at kSpRow): neighbour-of-Dirichlet band
   // entries zeroed, cross weights premultiplied by S, S^2, S, [S != 0] flag.
   double *row = spr + g * 16;
@@ -1413,11 +1397,18 @@ __global__ void var_tables_kernel(const HOpt *opts, const int64_t *row_opt,
   col[VT_V * vt_n] = v;
 }
 
-// Per option (one thread): Gz, the folded LU of I - tdt*A1 for S != 0 lines.
-__global__ void var_factor_kernel(HOpt *opts, int nopt, const double *__restrict__ vars,
-                                  double *vt, int64_t vt_n) {
-  const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= nopt) return;
+// Gz and the folded LU of I - tdt*A1 for S != 0 lines, one wave per option.
+// Bound by the pivots' serial chain: 64 rows at a time their band entries are
+// formed one row per lane and passed through LDS, every lane runs the chain on
+// broadcast reads, and each keeps the pivot of its row for the coalesced
+// results.  One thread per option, loading as it went, took 224 us for
+// one option of 1,024 rows (57 now) and 33 us for 150 (12 now).
+constexpr int kFactorRows = 64;
+__global__ void __launch_bounds__(64) var_factor_kernel(HOpt *opts,
+                                                        const double *__restrict__ vars, double *vt,
+                                                        int64_t vt_n) {
+  __shared__ __attribute__((aligned(16))) double rows[kFactorRows][4];
+  const int k = blockIdx.x, lane = threadIdx.x;
   HOpt o = opts[k];
   const int64_t n = o.nv;
   const double *m = vars + o.vo;
@@ -1444,45 +1435,94 @@ __global__ void var_factor_kernel(HOpt *opts, int nopt, const double *__restrict
   double *M = vt + VT_M * vt_n + o.vo, *RD = vt + VT_RD * vt_n + o.vo,
          *N = vt + VT_N * vt_n + o.vo;
   double rdprev = 0.0, cprev = 0.0;
-  for (int64_t j = 0; j < n; ++j) {
-    double a, b, c;
-    row(j, a, b, c);
+  for (int64_t j0 = 0; j0 < n; j0 += kFactorRows) {
+    const int64_t j = j0 + lane;
+    double a = 0.0, b = 1.0, c = 0.0;  // rows beyond the last one
+    if (j < n) row(j, a, b, c);
     if (j == n - 1) {
       a += f * b2;
       b += f * c2;
     }
-    const double l = a * rdprev;
-    const double rdj = 1.0 / (b - l * cprev);
-    M[j] = -l;
-    RD[j] = rdj;
-    N[j] = -c * rdj;
-    rdprev = rdj;
-    cprev = c;
+    __syncthreads();
+    rows[lane][0] = a;
+    rows[lane][1] = b;
+    rows[lane][2] = c;
+    __syncthreads();
+    const double before = rdprev;
+    double rd = 0.0;
+#pragma unroll 8
+    for (int q = 0; q < kFactorRows; ++q) {
+      const double l = rows[q][0] * rdprev;
+      rdprev = recip(rows[q][1] - l * cprev);
+      cprev = rows[q][2];
+      if (lane == q) rd = rdprev;
+    }
+    double rdup = __shfl_up(rd, 1, 64);
+    if (lane == 0) rdup = before;
+    if (j < n) {
+      M[j] = -(a * rdup);
+      RD[j] = rd;
+      N[j] = -c * rd;
+    }
   }
-  opts[k] = o;
+  if (lane == 0) opts[k] = o;
 }
 
-// One thread per spot line (option, column): pivots of I - tdt*A0 down the line.
-__global__ void spot_factor_kernel(Ctx c, const Tile *__restrict__ tiles, int ntiles,
-                                   double *rd0) {
-  const int64_t g = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  const int64_t tix = g / 64;
-  if (tix >= ntiles) return;
-  const Tile t = tiles[tix];
+// Pivots 1/b' of I - tdt*A0 on every spot line, one wave per 64 lines of an
+// option.  Bound by each line's serial chain (a mesh of 1,024 lines is 16
+// waves): the table rows, the same for all lanes, are fetched 64 at a time a
+// chunk ahead of the chain and read back from LDS, and the next rows' band
+// entries fill the chain's gaps.  Loading each row where it is used took 669
+// us on 2,048 x 1,024 nodes (212 now) and 50 us on 150 x 150 (17 now).
+__global__ void __launch_bounds__(64) spot_factor_kernel(Ctx c, const Tile *__restrict__ tiles,
+                                                         double *rd0) {
+  __shared__ __attribute__((aligned(16))) double rows[kFactorRows][8];
+  const Tile t = tiles[blockIdx.x];
   const HOpt o = c.opts[t.opt];
-  const int64_t j = t.start + (g % 64);
-  if (j >= o.nv) return;
-  const double v = c.vt[VT_V * c.vt_n + o.vo + j];
-  double *rd = rd0 + o.off;
-  double rdprev = 0.0, cprev = 0.0;
-  for (int64_t i = 0; i < o.nS; ++i) {
-    double a, b, cc;
-    li0_row(c, o, i, v, a, b, cc);
-    const double rdi = 1.0 / (b - (a * rdprev) * cprev);
-    rd[i * o.nv + j] = rdi;
-    rdprev = rdi;
-    cprev = cc;
+  const int lane = threadIdx.x;
+  const int64_t j = t.start + lane, n = o.nS;
+  const bool in = j < o.nv;
+  const double v = c.vt[VT_V * c.vt_n + o.vo + (in ? j : o.nv - 1)];
+  double *rd = rd0 + o.off + j;
+  double f[7];
+  auto fetch = [&](int64_t i) {  // table row i of this lane's (the last one beyond it)
+    const double *col = c.sp + o.so + (i < n ? i : n - 1);
+    f[0] = col[SP_PSUB * c.sp_n];
+    f[1] = col[SP_QSUB * c.sp_n];
+    f[2] = col[SP_PMID * c.sp_n];
+    f[3] = col[SP_QMID * c.sp_n];
+    f[4] = col[SP_PSUP * c.sp_n];
+    f[5] = col[SP_QSUP * c.sp_n];
+    f[6] = col[SP_S * c.sp_n];
+  };
+  // Row 0 is Dirichlet, and the last one of a barrier option: a = c = 0, b = 1.
+  double rdprev = 1.0, cprev = 0.0;
+  if (in) rd[0] = 1.0;
+  const int64_t last = o.barrier ? n - 1 : n;
+  fetch(1 + lane);
+  for (int64_t i0 = 1; i0 < last; i0 += kFactorRows) {
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < 7; ++q) rows[lane][q] = f[q];
+    __syncthreads();
+    fetch(i0 + kFactorRows + lane);
+    auto step = [&](int q) {
+      const double *w = rows[q];
+      const double c00 = c00_of(v, w[6]);
+      const double a = -o.tdt * band_add(w[0], w[1], c00);
+      const double b = 1.0 - o.tdt * band_add(w[2], w[3], c00);
+      rdprev = recip(b - (a * rdprev) * cprev);
+      cprev = -o.tdt * band_add(w[4], w[5], c00);
+      if (in) rd[(i0 + q) * o.nv] = rdprev;
+    };
+    if (last - i0 >= kFactorRows) {
+#pragma unroll 8
+      for (int q = 0; q < kFactorRows; ++q) step(q);
+    } else {
+      for (int q = 0; q < (int)(last - i0); ++q) step(q);
+    }
   }
+  if (o.barrier && in) rd[(n - 1) * o.nv] = 1.0 / (1.0 - (0.0 * rdprev) * cprev);
 }
 
 // Step sizes of every option from the scheme's theta and the dt multiplier,
@@ -2006,11 +2046,11 @@ int refactor(fdadi_hb *hb, hipStream_t s, const double *d_theta = nullptr,
                      hb->dt_scale, (int)(hb->scheme == FDADI_SCHEME_IMPLICIT),
                      reuse ? nullptr : hb->d_slots);
   FDADI_CHECK_LAUNCH();
-  hipLaunchKernelGGL(var_factor_kernel, dim3(grid_for(hb->nopt, 64)), dim3(64), 0, s, hb->d_opts,
-                     hb->nopt, hb->d_vars, hb->d_vt, hb->vt_n);
+  hipLaunchKernelGGL(var_factor_kernel, dim3(hb->nopt), dim3(64), 0, s, hb->d_opts, hb->d_vars,
+                     hb->d_vt, hb->vt_n);
   FDADI_CHECK_LAUNCH();
   hipLaunchKernelGGL(spot_factor_kernel, dim3(hb->nftiles), dim3(64), 0, s, ctx_of(hb),
-                     hb->d_ftiles, hb->nftiles, hb->d_rd0);
+                     hb->d_ftiles, hb->d_rd0);
   FDADI_CHECK_LAUNCH();
   if (!dev && !capturing) FDADI_TRY_HIP(hipStreamSynchronize(s));
   return FDADI_OK;
