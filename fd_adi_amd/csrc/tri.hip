@@ -97,170 +97,244 @@ __global__ void tri_apply_kernel(TriView o, const double *__restrict__ x,
   y[sidx(o, line, pos)] = v;
 }
 
-// Thomas sweep (no pivoting), one thread per line, one wave per 64
-// consecutive lines.  The bands, the right-hand side, the modified
-// super-diagonal (`cp`, in scratch) and the forward-substituted values
-// (kept in place in v) move between global memory and LDS in tiles of 64
-// lines x kSolveChunk positions with coalesced accesses -- 128-byte runs of
-// one line for line-major arrays, 64 consecutive lines of one position for
-// the strided state of axis 0 -- and each thread runs its line's
-// recurrences out of the LDS tile (odd pitch: no bank conflicts).  Rows 0
-// and n-1 (with their fold entries) are read directly, once per line.
-constexpr int kSolveChunk = 16;
+// Thomas sweep (no pivoting), one thread per line, kSolveLines lines per
+// work-group.  Bound by the lines' serial chains, so the whole work-group moves
+// the data: 64 rows at a time the bands and the right-hand side go to LDS (the
+// next chunk's loads are under way while the chains run), rows of one line
+// together for line-major arrays, the lines of one position together for the
+// strided state of axis 0, and each chain runs out of LDS eight rows at a time
+// (odd pitch: no bank conflicts).  Few lines per work-group, for there are few
+// lines: 151 of them are 19 work-groups.  The modified super-diagonal and the
+// forward-substituted values stay in LDS where lines are short (KEEP);
+// otherwise they go to scratch (`cpg`) and v, chunk by chunk.  One wave for 64
+// lines, which staged 16 rows at a time before each stretch of the chain, took
+// 121 us for 151 lines of 81 and 212 us for 81 lines of 151 (13 and 19 now).
+constexpr int kSolveLines = 8, kSolveChunk = 64, kSolveThreads = 256;
+constexpr int kSolvePer = kSolveLines * kSolveChunk / kSolveThreads;  // elements per thread
 constexpr int kSolvePitch = kSolveChunk + 1;
+constexpr int kKeepRows = 384;  // 8 lines x 385 x 2 values: 49 KB
+static_assert(kKeepRows % kSolveChunk == 0, "whole chunks");
 
-__device__ __forceinline__ void tile_index(const TriView &o, int64_t L0, int64_t p0, int e,
-                                           bool state, int &l, int &p, int64_t &g, bool &ok) {
-  const int64_t n = o.bl;
-  if (state && o.axis == 0) {  // position-major: 64 lines of one position per load
-    p = e / 64;
-    l = e % 64;
-  } else {  // line-major: runs of kSolveChunk positions of one line
+// Element e of the chunk of rows from p0: line l and row p of the tile, g in
+// the array (the state, or a line-major one); false outside of the operator.
+__device__ __forceinline__ bool tile_index(const TriView &o, int64_t L0, int64_t p0, int e,
+                                           bool state, int &l, int &p, int64_t &g) {
+  if (state && o.axis == 0) {
+    p = e / kSolveLines;
+    l = e % kSolveLines;
+  } else {
     l = e / kSolveChunk;
     p = e % kSolveChunk;
   }
   const int64_t line = L0 + l, pos = p0 + p;
-  ok = line < o.blocks && pos < n;
-  g = ok ? (state ? sidx(o, line, pos) : line * n + pos) : 0;
+  g = state ? sidx(o, line, pos) : line * o.bl + pos;
+  return line < o.blocks && pos < o.bl;
 }
 
-__global__ void __launch_bounds__(64)
+template <bool KEEP>
+__global__ void __launch_bounds__(kSolveThreads)
 tri_solve_kernel(TriView o, double *__restrict__ v, double *__restrict__ cpg) {
-  __shared__ double ta[64 * kSolvePitch], tb[64 * kSolvePitch], tc[64 * kSolvePitch],
-      td[64 * kSolvePitch];
+  constexpr int CP = KEEP ? kKeepRows + 1 : kSolvePitch;
+  __shared__ double ta[kSolveLines * kSolvePitch], tb[kSolveLines * kSolvePitch],
+      tc[kSolveLines * CP], td[kSolveLines * CP];
   const int t = threadIdx.x;
-  const int64_t L0 = (int64_t)blockIdx.x * 64, line = L0 + t, n = o.bl, base = line * n;
-  const bool live = line < o.blocks;
-  auto rhs_at = [&](int64_t p) {
-    double d = xf(o, v, line, p);
-    if (o.has_residual) d -= o.R[base + p];
-    return d;
+  const int64_t L0 = (int64_t)blockIdx.x * kSolveLines, line = L0 + t, n = o.bl;
+  const bool chain = t < kSolveLines && line < o.blocks;
+  double ra[kSolvePer], rb[kSolvePer], rc[kSolvePer], rr[kSolvePer], rx[kSolvePer];
+  auto fetch = [&](int64_t p0) {
+#pragma unroll
+    for (int q = 0; q < kSolvePer; ++q) {
+      int l, p;
+      int64_t g;
+      ra[q] = rb[q] = rc[q] = rr[q] = rx[q] = 0.0;
+      if (tile_index(o, L0, p0, t + kSolveThreads * q, false, l, p, g)) {
+        ra[q] = o.sub[g];
+        rb[q] = o.mid[g];
+        rc[q] = o.sup[g];
+        if (o.has_residual) rr[q] = o.R[g];
+      }
+      if (tile_index(o, L0, p0, t + kSolveThreads * q, true, l, p, g))
+        rx[q] = xf(o, v, L0 + l, p0 + p);
+    }
   };
-  // Row 0 (with top fold) and the last row (with bottom fold), per line.
-  double b0 = 0.0, c0 = 0.0, d0 = 0.0, an = 0.0, bn = 0.0, fbot = 0.0;
-  if (live) {
-    b0 = o.mid[base];
-    c0 = o.sup[base];
-    d0 = rhs_at(0);
-    if (o.top_status == FDADI_FOLDED) {
-      d0 += o.top[line] * rhs_at(1);
-    } else if (o.top_status == FDADI_CAN_FOLD) {
-      const double c1 = o.sup[base + 1];
-      const double f = c1 == 0 ? 0.0 : -o.top[line] / c1;
-      b0 += f * o.sub[base + 1];
-      c0 += f * o.mid[base + 1];
-      d0 += f * rhs_at(1);
+  // The fetched chunk into LDS, the right-hand side as x - R.
+  auto stage = [&](int off) {
+    int l, p;
+    int64_t g;
+#pragma unroll
+    for (int q = 0; q < kSolvePer; ++q) {
+      tile_index(o, L0, 0, t + kSolveThreads * q, false, l, p, g);
+      ta[l * kSolvePitch + p] = ra[q];
+      tb[l * kSolvePitch + p] = rb[q];
+      tc[l * CP + off + p] = rc[q];
+      if (o.has_residual) td[l * CP + off + p] = rr[q];
     }
-    an = o.sub[base + n - 1];
-    bn = o.mid[base + n - 1];
-    if (o.bottom_status == FDADI_FOLDED) {
-      fbot = o.bottom[line];
-    } else if (o.bottom_status == FDADI_CAN_FOLD) {
-      const double a = o.sub[base + n - 2];
-      fbot = a == 0 ? 0.0 : -o.bottom[line] / a;
-      an += fbot * o.mid[base + n - 2];
-      bn += fbot * o.sup[base + n - 2];
+    if (o.has_residual) __syncthreads();
+#pragma unroll
+    for (int q = 0; q < kSolvePer; ++q) {
+      tile_index(o, L0, 0, t + kSolveThreads * q, true, l, p, g);
+      double *slot = &td[l * CP + off + p];
+      *slot = o.has_residual ? rx[q] - *slot : rx[q];
     }
-  }
-  // Forward elimination, chunk by chunk.
+  };
+  // The chunk's values, and with cp its modified super-diagonal, to memory.
+  auto put = [&](int64_t p0, int off, bool cp) {
+#pragma unroll
+    for (int q = 0; q < kSolvePer; ++q) {
+      int l, p;
+      int64_t g;
+      if (cp && tile_index(o, L0, p0, t + kSolveThreads * q, false, l, p, g))
+        cpg[g] = tc[l * CP + off + p];
+      if (tile_index(o, L0, p0, t + kSolveThreads * q, true, l, p, g)) v[g] = td[l * CP + off + p];
+    }
+  };
+
   double cprev = 0.0, dprev = 0.0, dnm2 = 0.0;
+  double pa = 0.0, pb = 0.0, pc = 0.0;  // bands of the row before, as they are
+  const double *la = ta + t * kSolvePitch, *lb = tb + t * kSolvePitch;  // this line's
+  fetch(0);
   for (int64_t p0 = 0; p0 < n; p0 += kSolveChunk) {
-    for (int e = t; e < 64 * kSolveChunk; e += 64) {
-      int l, p;
-      int64_t g;
-      bool ok;
-      tile_index(o, L0, p0, e, false, l, p, g, ok);
-      ta[l * kSolvePitch + p] = ok ? o.sub[g] : 0.0;
-      tb[l * kSolvePitch + p] = ok ? o.mid[g] : 0.0;
-      tc[l * kSolvePitch + p] = ok ? o.sup[g] : 0.0;
-      if (o.has_residual) td[l * kSolvePitch + p] = ok ? -o.R[g] : 0.0;
-    }
+    const int off = KEEP ? (int)p0 : 0;
+    double *lc = tc + t * CP + off, *ld = td + t * CP + off;
     __syncthreads();
-    for (int e = t; e < 64 * kSolveChunk; e += 64) {
-      int l, p;
-      int64_t g;
-      bool ok;
-      tile_index(o, L0, p0, e, true, l, p, g, ok);
-      const int64_t ln = L0 + l, pos = p0 + p;
-      double x = 0.0;
-      if (ok) {
-        if (pos == 0 && o.has_low) x = o.low[ln];
-        else if (pos == n - 1 && o.has_high) x = o.high[ln];
-        else x = v[g];
-      }
-      // rhs = x - R (the R tile holds -R when the residual is on)
-      double &slot = td[l * kSolvePitch + p];
-      slot = o.has_residual ? x + slot : x;
-    }
+    stage(off);
     __syncthreads();
-    if (live) {
-      for (int k = 0; k < kSolveChunk && p0 + k < n; ++k) {
-        const int64_t pos = p0 + k;
-        double *ck = &tc[t * kSolvePitch + k], *dk = &td[t * kSolvePitch + k];
-        if (pos == 0) {
-          cprev = c0 / b0;
-          dprev = d0 / b0;
-        } else {
-          double a, b, c, d;
-          if (pos == n - 1) {
-            d = *dk + fbot * dnm2;
-            a = an; b = bn; c = 0.0;
-          } else {
-            d = *dk;
-            if (pos == n - 2) dnm2 = d;
-            a = ta[t * kSolvePitch + k]; b = tb[t * kSolvePitch + k]; c = *ck;
-          }
-          const double m = 1.0 / (b - a * cprev);
-          cprev = c * m;
-          dprev = (d - a * dprev) * m;
+    if (p0 + kSolveChunk < n) fetch(p0 + kSolveChunk);
+    if (chain) {
+      int k = 0;
+      if (p0 == 0) {  // row 0, with the top fold
+        double b0 = lb[0], c0 = lc[0], d0 = ld[0];
+        pa = la[0];
+        pb = b0;
+        pc = c0;
+        if (o.top_status == FDADI_FOLDED) {
+          d0 += o.top[line] * ld[1];
+        } else if (o.top_status == FDADI_CAN_FOLD) {
+          const double c1 = lc[1];
+          const double f = c1 == 0 ? 0.0 : -o.top[line] / c1;
+          b0 += f * la[1];
+          c0 += f * lb[1];
+          d0 += f * ld[1];
         }
-        *ck = cprev;
-        *dk = dprev;
+        cprev = c0 / b0;
+        dprev = d0 / b0;
+        lc[0] = cprev;
+        ld[0] = dprev;
+        k = 1;
+      }
+      auto eliminate = [&](double a, double b, double c, double d) {
+        const double m = 1.0 / (b - a * cprev);
+        cprev = c * m;
+        dprev = (d - a * dprev) * m;
+      };
+      const int end = n - 1 - p0 < kSolveChunk ? (int)(n - 1 - p0) : kSolveChunk;
+      for (; k + 8 <= end; k += 8) {
+        double a[8], b[8], c[8], d[8];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+          a[q] = la[k + q];
+          b[q] = lb[k + q];
+          c[q] = lc[k + q];
+          d[q] = ld[k + q];
+        }
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+          eliminate(a[q], b[q], c[q], d[q]);
+          lc[k + q] = cprev;
+          ld[k + q] = dprev;
+        }
+        pa = a[7];
+        pb = b[7];
+        pc = c[7];
+        dnm2 = d[7];
+      }
+      for (; k < end; ++k) {
+        pa = la[k];
+        pb = lb[k];
+        pc = lc[k];
+        dnm2 = ld[k];
+        eliminate(pa, pb, pc, dnm2);
+        lc[k] = cprev;
+        ld[k] = dprev;
+      }
+      if (k < kSolveChunk && k == n - 1 - p0) {  // the last row, with the bottom fold
+        double an = la[k], bn = lb[k], fbot = 0.0;
+        if (o.bottom_status == FDADI_FOLDED) {
+          fbot = o.bottom[line];
+        } else if (o.bottom_status == FDADI_CAN_FOLD) {
+          fbot = pa == 0 ? 0.0 : -o.bottom[line] / pa;
+          an += fbot * pb;
+          bn += fbot * pc;
+        }
+        eliminate(an, bn, 0.0, ld[k] + fbot * dnm2);
+        lc[k] = cprev;
+        ld[k] = dprev;
       }
     }
-    __syncthreads();
-    for (int e = t; e < 64 * kSolveChunk; e += 64) {
-      int l, p;
-      int64_t g;
-      bool ok;
-      tile_index(o, L0, p0, e, false, l, p, g, ok);
-      if (ok) cpg[g] = tc[l * kSolvePitch + p];
-      tile_index(o, L0, p0, e, true, l, p, g, ok);
-      if (ok) v[g] = td[l * kSolvePitch + p];
+    if (!KEEP) {
+      __syncthreads();
+      put(p0, 0, true);
     }
-    __syncthreads();
   }
-  // Back substitution, chunks from the last; x(n-1) = dprev.
+  // Back substitution from row n - 2; x(n-1) = dprev, already in place.
   double x = dprev;
+  auto back = [&](double *lc, double *ld, int k) {  // rows k .. 0 of the pointers
+    for (; k >= 7; k -= 8) {
+      double c[8], d[8];
+#pragma unroll
+      for (int q = 0; q < 8; ++q) {
+        c[q] = lc[k - q];
+        d[q] = ld[k - q];
+      }
+#pragma unroll
+      for (int q = 0; q < 8; ++q) {
+        x = d[q] - c[q] * x;
+        ld[k - q] = x;
+      }
+    }
+    for (; k >= 0; --k) {
+      x = ld[k] - lc[k] * x;
+      ld[k] = x;
+    }
+  };
+  if (KEEP) {
+    if (chain) back(tc + t * CP, td + t * CP, (int)n - 2);
+    __syncthreads();
+    for (int64_t p0 = 0; p0 < n; p0 += kSolveChunk) put(p0, (int)p0, false);
+    return;
+  }
+  // The last chunk is still in LDS; each thread reads back what it wrote.
   const int64_t last0 = (n - 1) / kSolveChunk * kSolveChunk;
-  for (int64_t p0 = last0; p0 >= 0; p0 -= kSolveChunk) {
-    for (int e = t; e < 64 * kSolveChunk; e += 64) {
+  auto fetch_back = [&](int64_t p0) {
+#pragma unroll
+    for (int q = 0; q < kSolvePer; ++q) {
       int l, p;
       int64_t g;
-      bool ok;
-      tile_index(o, L0, p0, e, false, l, p, g, ok);
-      tc[l * kSolvePitch + p] = ok ? cpg[g] : 0.0;
-      tile_index(o, L0, p0, e, true, l, p, g, ok);
-      td[l * kSolvePitch + p] = ok ? v[g] : 0.0;
+      rc[q] = rx[q] = 0.0;
+      if (tile_index(o, L0, p0, t + kSolveThreads * q, false, l, p, g)) rc[q] = cpg[g];
+      if (tile_index(o, L0, p0, t + kSolveThreads * q, true, l, p, g)) rx[q] = v[g];
     }
-    __syncthreads();
-    if (live) {
-      for (int k = kSolveChunk - 1; k >= 0; --k) {
-        const int64_t pos = p0 + k;
-        if (pos > n - 2) continue;  // x(n-1) is dprev, already in place
-        x = td[t * kSolvePitch + k] - tc[t * kSolvePitch + k] * x;
-        td[t * kSolvePitch + k] = x;
+  };
+  for (int64_t p0 = last0; p0 >= 0; p0 -= kSolveChunk) {
+    if (p0 != last0) {
+      __syncthreads();
+#pragma unroll
+      for (int q = 0; q < kSolvePer; ++q) {
+        int l, p;
+        int64_t g;
+        tile_index(o, L0, 0, t + kSolveThreads * q, false, l, p, g);
+        tc[l * CP + p] = rc[q];
+        tile_index(o, L0, 0, t + kSolveThreads * q, true, l, p, g);
+        td[l * CP + p] = rx[q];
       }
     }
     __syncthreads();
-    for (int e = t; e < 64 * kSolveChunk; e += 64) {
-      int l, p;
-      int64_t g;
-      bool ok;
-      tile_index(o, L0, p0, e, true, l, p, g, ok);
-      if (ok) v[g] = td[l * kSolvePitch + p];
-    }
+    if (p0 > 0) fetch_back(p0 - kSolveChunk);
+    if (chain)
+      back(tc + t * CP, td + t * CP,
+           n - 2 - p0 < kSolveChunk - 1 ? (int)(n - 2 - p0) : kSolveChunk - 1);
     __syncthreads();
+    put(p0, 0, false);
   }
 }
 
@@ -681,8 +755,13 @@ int fdadi_tri_solve(const fdadi_tri *op, double *d_v, int64_t n, void *stream) {
   FDADI_REQUIRE(n == op->rows, FDADI_ERR_ARG,
                 "fdadi_tri_solve: vector size " + std::to_string(n) +
                     " != operator rows " + std::to_string(op->rows));
-  hipLaunchKernelGGL(tri_solve_kernel, dim3(grid_for(op->blocks, 64)), dim3(64), 0,
-                     as_stream(stream), view_of(op), d_v, op->scratch);
+  const dim3 grid(grid_for(op->blocks, kSolveLines));
+  if (op->block_len <= kKeepRows)
+    hipLaunchKernelGGL(tri_solve_kernel<true>, grid, dim3(kSolveThreads), 0, as_stream(stream),
+                       view_of(op), d_v, op->scratch);
+  else
+    hipLaunchKernelGGL(tri_solve_kernel<false>, grid, dim3(kSolveThreads), 0, as_stream(stream),
+                       view_of(op), d_v, op->scratch);
   FDADI_CHECK_LAUNCH();
   return FDADI_OK;
 }
