@@ -405,6 +405,22 @@ class BandedOperator(object):
         _lib.call("fdadi_array_copy", sa_U.p, tmp.ptr, n, s)
         return sa_U
 
+    def apply_to_(self, sa_V, sa_U):
+        """sa_U = A sa_V on device arrays, without the copies of ``apply_``."""
+        if sa_U.size != sa_V.size:
+            raise ValueError("apply_to_: size mismatch (%d != %d)" % (sa_U.size, sa_V.size))
+        name, h = ("fdadi_tri_apply", self._tri) if self._tri is not None else \
+            ("fdadi_cross_apply", self._csr)
+        _lib.call(name, h, sa_V.p, sa_U.p, sa_V.size, _lib.default_stream())
+
+    def apply_add_(self, sa_V, sa_U, minus=False):
+        """sa_U += A sa_V (-= with ``minus``) on device arrays, in one launch."""
+        if sa_U.size != sa_V.size:
+            raise ValueError("apply_add_: size mismatch (%d != %d)" % (sa_U.size, sa_V.size))
+        name, h = ("fdadi_tri_apply_add", self._tri) if self._tri is not None else \
+            ("fdadi_cross_apply_add", self._csr)
+        _lib.call(name, h, sa_V.p, sa_U.p, sa_V.size, int(minus), _lib.default_stream())
+
     def apply(self, V, overwrite=False):
         """Wrapper for CPU based data."""
         sa_V = SizedArrayPtr(np.asarray(V), "sa_V apply")

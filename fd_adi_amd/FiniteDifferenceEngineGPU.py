@@ -274,8 +274,7 @@ class FiniteDifferenceEngineADI(FiniteDifferenceEngine):
         U = SizedArrayPtr().alloc(V.size)
         for _ in range(int(n)):
             if cross is not None:
-                U.copy_from(V)
-                cross.apply_(U, overwrite=True)
+                cross.apply_to_(V, U)
                 V.pluseq(U)
             for L in Lis:
                 L.solve_(V, overwrite=True)
@@ -298,16 +297,11 @@ class FiniteDifferenceEngineADI(FiniteDifferenceEngine):
             if L.is_foldable():
                 L.diagonalize()
         Y = V.copy(True)
-        X = SizedArrayPtr().alloc(V.size)
         for _ in range(int(n)):
             for L in Firsts:
-                X.copy_from(Y)
-                L.apply_(X, overwrite=True)
-                V.pluseq(X)
+                L.apply_add_(Y, V)
             for Le, Li in zip(Les, Lis):
-                X.copy_from(Y)
-                Le.apply_(X, overwrite=True)
-                V.minuseq(X)
+                Le.apply_add_(Y, V, minus=True)
                 Li.solve_(V, overwrite=True)
             Y.copy_from(V)
         _lib.sync()
@@ -321,32 +315,23 @@ class FiniteDifferenceEngineADI(FiniteDifferenceEngine):
         for L in itertools.chain(Les, Lis, Firsts):
             if L.is_foldable():
                 L.diagonalize()
-        X = SizedArrayPtr().alloc(V.size)
         Y = SizedArrayPtr().alloc(V.size)
         Z = SizedArrayPtr().alloc(V.size)
         for _ in range(int(n)):
             Y.copy_from(V)
             for L in Firsts:
-                X.copy_from(Y)
-                L.apply_(X, overwrite=True)
-                V.pluseq(X)
+                L.apply_add_(Y, V)
             Z.copy_from(V)
             for Le, Li in zip(Les, Lis):
-                X.copy_from(Y)
-                Le.apply_(X, overwrite=True)
-                Z.minuseq(X)
+                Le.apply_add_(Y, Z, minus=True)
                 Li.solve_(Z, overwrite=True)
             Y.minuseq_over2(Z)
             for L in Firsts:
                 L.enable_residual(False)
-                X.copy_from(Y)
-                L.apply_(X, overwrite=True)
-                V.minuseq(X)
+                L.apply_add_(Y, V, minus=True)
                 L.enable_residual(True)
             for Le, Li in zip(Les, Lis):
-                X.copy_from(Z)
-                Le.apply_(X, overwrite=True)
-                V.minuseq(X)
+                Le.apply_add_(Z, V, minus=True)
                 Li.solve_(V, overwrite=True)
         _lib.sync()
 
@@ -361,33 +346,25 @@ class FiniteDifferenceEngineADI(FiniteDifferenceEngine):
         for _ in range(int(n)):
             Y.copy_from(V)
             for L in Firsts:
-                X.copy_from(V)
-                L.apply_(X, overwrite=True)
-                Y.pluseq(X)
+                L.apply_add_(V, Y)
             Y0.copy_from(Y)
             for Le, Li in zip(Les, Lis):
-                X.copy_from(V)
-                Le.apply_(X, overwrite=True)
-                Y.minuseq(X)
+                Le.apply_add_(V, Y, minus=True)
                 Li.solve_(Y, overwrite=True)
             D.copy_from(Y)
             D.minuseq(V)              # D = Y2 - V
             Y.copy_from(Y0)
             if cross is not None:
-                X.copy_from(D)
-                cross.apply_(X, overwrite=True)
+                cross.apply_to_(D, X)
                 X.timeseq_scalar_from_host(th * dt_h if modified else 0.5 * dt_h)
                 Y.pluseq(X)
             if modified:
                 for L in Firsts:      # (1/2 - theta) F(Y2 - V), residual included
-                    X.copy_from(D)
-                    L.apply_(X, overwrite=True)
+                    L.apply_to_(D, X)
                     X.timeseq_scalar_from_host(0.5 - th)
                     Y.pluseq(X)
             for Le, Li in zip(Les, Lis):
-                X.copy_from(V)
-                Le.apply_(X, overwrite=True)
-                Y.minuseq(X)
+                Le.apply_add_(V, Y, minus=True)
                 Li.solve_(Y, overwrite=True)
             V.copy_from(Y)
         _lib.sync()

@@ -73,6 +73,7 @@ _SIGS = {
     "fdadi_tri_set_flags": (c_int, [c_vp, c_int, c_int, c_int]),
     "fdadi_tri_read": (c_int, [c_vp] + [c_vp] * 9),
     "fdadi_tri_apply": (c_int, [c_vp, c_vp, c_vp, c_i64, c_vp]),
+    "fdadi_tri_apply_add": (c_int, [c_vp, c_vp, c_vp, c_i64, c_i32, c_vp]),
     "fdadi_tri_solve": (c_int, [c_vp, c_vp, c_i64, c_vp]),
     "fdadi_tri_add_operator": (c_int, [c_vp, c_vp, c_vp]),
     "fdadi_tri_add_scalar": (c_int, [c_vp, c_double, c_vp]),
@@ -90,6 +91,7 @@ _SIGS = {
     "fdadi_cross_info": (c_int, [c_vp, _P(c_i64), _P(c_i64)]),
     "fdadi_cross_read": (c_int, [c_vp, c_vp, c_vp]),
     "fdadi_cross_apply": (c_int, [c_vp, c_vp, c_vp, c_i64, c_vp]),
+    "fdadi_cross_apply_add": (c_int, [c_vp, c_vp, c_vp, c_i64, c_i32, c_vp]),
     "fdadi_cross_scale": (c_int, [c_vp, c_vp, c_i64, c_vp]),
     "fdadi_cross_scale_scalar": (c_int, [c_vp, c_double, c_vp]),
     "fdadi_heston_coefficients": (c_int, [c_int, c_vp, c_i64, c_vp, c_i64, c_vp, c_vp, c_vp]),

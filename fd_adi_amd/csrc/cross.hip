@@ -55,6 +55,8 @@ __global__ void cross_for_vector_kernel(const double *__restrict__ m0, int64_t n
     }
 }
 
+// y = A x (SIGN 0), or y += A x / y -= A x.
+template <int SIGN>
 __global__ void cross_apply_kernel(const double *__restrict__ bands, const double *__restrict__ R,
                                    int64_t n0, int64_t n1, const double *__restrict__ x,
                                    double *__restrict__ y) {
@@ -73,7 +75,11 @@ __global__ void cross_apply_kernel(const double *__restrict__ bands, const doubl
       acc += bands[k * N + r] * x[ii * n1 + jj];
     }
   }
-  y[r] = acc + R[r];
+  const double v = acc + R[r];
+  {
+#pragma clang fp contract(off)
+    y[r] = SIGN == 0 ? v : SIGN > 0 ? y[r] + v : y[r] - v;
+  }
 }
 
 // Scale by vec tiled over the rows, or by the scalar `value` when vec is null.
@@ -256,8 +262,26 @@ int fdadi_cross_apply(const fdadi_cross *op, const double *d_x, double *d_y, int
                 "fdadi_cross_apply: vector size " + std::to_string(n) + " != operator rows " +
                     std::to_string(op->N));
   FDADI_REQUIRE(d_x != d_y, FDADI_ERR_ARG, "fdadi_cross_apply: output must not alias input");
-  hipLaunchKernelGGL(cross_apply_kernel, dim3(grid_for(op->N, kBlock)), dim3(kBlock), 0,
+  hipLaunchKernelGGL(cross_apply_kernel<0>, dim3(grid_for(op->N, kBlock)), dim3(kBlock), 0,
                      as_stream(stream), op->bands, op->R, op->n0, op->n1, d_x, d_y);
+  FDADI_CHECK_LAUNCH();
+  return FDADI_OK;
+}
+
+int fdadi_cross_apply_add(const fdadi_cross *op, const double *d_x, double *d_y, int64_t n,
+                          int32_t minus, void *stream) {
+  FDADI_REQUIRE(op && d_x && d_y, FDADI_ERR_ARG, "fdadi_cross_apply_add: null argument");
+  FDADI_REQUIRE(n == op->N, FDADI_ERR_ARG,
+                "fdadi_cross_apply_add: vector size " + std::to_string(n) + " != operator rows " +
+                    std::to_string(op->N));
+  FDADI_REQUIRE(d_x != d_y, FDADI_ERR_ARG, "fdadi_cross_apply_add: output must not alias input");
+  const dim3 grid(grid_for(op->N, kBlock));
+  if (minus)
+    hipLaunchKernelGGL(cross_apply_kernel<-1>, grid, dim3(kBlock), 0, as_stream(stream), op->bands,
+                       op->R, op->n0, op->n1, d_x, d_y);
+  else
+    hipLaunchKernelGGL(cross_apply_kernel<1>, grid, dim3(kBlock), 0, as_stream(stream), op->bands,
+                       op->R, op->n0, op->n1, d_x, d_y);
   FDADI_CHECK_LAUNCH();
   return FDADI_OK;
 }

@@ -81,6 +81,9 @@ __device__ double row_dot(const TriView &o, const double *x, int64_t line, int64
   return acc;
 }
 
+// y = A x (SIGN 0), or y += A x / y -= A x, which saves a scheme's stage the
+// product's copy and the sum's pass (bit for bit their result).
+template <int SIGN>
 __global__ void tri_apply_kernel(TriView o, const double *__restrict__ x,
                                  double *__restrict__ y) {
   const int64_t r = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
@@ -94,7 +97,11 @@ __global__ void tri_apply_kernel(TriView o, const double *__restrict__ x,
   if (pos == 0 && o.top_status == FDADI_FOLDED)
     v -= o.top[line] * row_dot(o, x, line, 1);
   if (o.has_residual) v += o.R[r];
-  y[sidx(o, line, pos)] = v;
+  double &out = y[sidx(o, line, pos)];
+  {
+#pragma clang fp contract(off)
+    out = SIGN == 0 ? v : SIGN > 0 ? out + v : out - v;
+  }
 }
 
 // Thomas sweep (no pivoting), one thread per line, kSolveLines lines per
@@ -744,8 +751,26 @@ int fdadi_tri_apply(const fdadi_tri *op, const double *d_x, double *d_y, int64_t
                 "fdadi_tri_apply: vector size " + std::to_string(n) +
                     " != operator rows " + std::to_string(op->rows));
   FDADI_REQUIRE(d_x != d_y, FDADI_ERR_ARG, "fdadi_tri_apply: output must not alias input");
-  hipLaunchKernelGGL(tri_apply_kernel, dim3(grid_for(op->rows, kBlock)), dim3(kBlock), 0,
+  hipLaunchKernelGGL(tri_apply_kernel<0>, dim3(grid_for(op->rows, kBlock)), dim3(kBlock), 0,
                      as_stream(stream), view_of(op), d_x, d_y);
+  FDADI_CHECK_LAUNCH();
+  return FDADI_OK;
+}
+
+int fdadi_tri_apply_add(const fdadi_tri *op, const double *d_x, double *d_y, int64_t n,
+                        int32_t minus, void *stream) {
+  FDADI_REQUIRE(op && d_x && d_y, FDADI_ERR_ARG, "fdadi_tri_apply_add: null argument");
+  FDADI_REQUIRE(n == op->rows, FDADI_ERR_ARG,
+                "fdadi_tri_apply_add: vector size " + std::to_string(n) +
+                    " != operator rows " + std::to_string(op->rows));
+  FDADI_REQUIRE(d_x != d_y, FDADI_ERR_ARG, "fdadi_tri_apply_add: output must not alias input");
+  const dim3 grid(grid_for(op->rows, kBlock));
+  if (minus)
+    hipLaunchKernelGGL(tri_apply_kernel<-1>, grid, dim3(kBlock), 0, as_stream(stream), view_of(op),
+                       d_x, d_y);
+  else
+    hipLaunchKernelGGL(tri_apply_kernel<1>, grid, dim3(kBlock), 0, as_stream(stream), view_of(op),
+                       d_x, d_y);
   FDADI_CHECK_LAUNCH();
   return FDADI_OK;
 }

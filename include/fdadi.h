@@ -119,6 +119,9 @@ int fdadi_tri_read(const fdadi_tri *op, double *sup, double *mid, double *sub, d
  * alias d_x.  A CAN_FOLD (unfolded) operator is applied with its +-2 entries. */
 int fdadi_tri_apply(const fdadi_tri *op, const double *d_x, double *d_y, int64_t n,
                     void *stream);
+/* d_y += A x (+R), or -= with minus: apply and the elementwise sum in one pass. */
+int fdadi_tri_apply_add(const fdadi_tri *op, const double *d_x, double *d_y, int64_t n,
+                        int32_t minus, void *stream);
 /* solve, _TriBandedOperatorGPU.cu:719-770: d_v <- A^-1 (v - R) per grid line,
  * Dirichlet rows forced, RHS folded as needed (replaces
  * cusparseDgtsvStridedBatch and the transposes). */
@@ -155,6 +158,9 @@ int fdadi_cross_read(const fdadi_cross *op, double *bands, double *R);
 /* apply, _CSRBandedOperatorGPU.cu:340-426 (replaces cusparseDcsrmv). */
 int fdadi_cross_apply(const fdadi_cross *op, const double *d_x, double *d_y, int64_t n,
                       void *stream);
+/* d_y += A x (+R), or -= with minus. */
+int fdadi_cross_apply_add(const fdadi_cross *op, const double *d_x, double *d_y, int64_t n,
+                          int32_t minus, void *stream);
 /* vectorized_scale, _CSRBandedOperatorGPU.cu:442-480. */
 int fdadi_cross_scale(fdadi_cross *op, const double *d_vec, int64_t vsize, void *stream);
 int fdadi_cross_scale_scalar(fdadi_cross *op, double value, void *stream);
