@@ -25,6 +25,93 @@ struct FNode {
   int32_t feature, left, right, leaf;
 };
 
+// Trees of at most kTreeNodes nodes (64 leaves: the gate's models are grown to
+// 63) over at most kTreeFeat features, in LDS.  A
+// walk is a chain of dependent reads, node then feature: from memory one wave
+// per SIMD waited out each of them (234 us for 50,000 rows, 41 now).  Here a
+// work-group takes 128 rows, their features in LDS (a lane's own bank whatever
+// feature it asks for), and stages kTreeBatch trees at a time, 12 bytes a node,
+// the next batch's loads under way; each wave walks four trees of its 64 rows
+// side by side, and the leaves are added in the order of the trees.
+constexpr int kTreeNodes = 128, kTreeFeat = 16, kTreeBatch = 16, kTreeRows = 128;
+constexpr int kTreeThreads = 512, kTreeIlp = 4;
+constexpr uint32_t kTreeLeaf = 0x80000000u;  // else feature << 16 | right << 8 | left
+static_assert(kTreeBatch == kTreeIlp * (kTreeThreads / 64) / (kTreeRows / 64), "waves' trees");
+
+// thr: kTreeNodes values per tree (a leaf's is its value), meta likewise; both
+// padded to whole batches with leaves.
+__global__ void __launch_bounds__(kTreeThreads)
+forest_tile_kernel(const double *__restrict__ thr, const uint32_t *__restrict__ meta, int ntrees,
+                   double base, const double *__restrict__ X, int64_t n, int nfeat,
+                   double *__restrict__ out) {
+  __shared__ __attribute__((aligned(16))) double sthr[kTreeBatch * kTreeNodes];
+  __shared__ __attribute__((aligned(16))) uint32_t smeta[kTreeBatch * kTreeNodes];
+  __shared__ double sx[kTreeFeat * kTreeRows], leaf[kTreeBatch * kTreeRows];
+  const int tid = threadIdx.x, wave = tid / 64;
+  const int64_t row0 = (int64_t)blockIdx.x * kTreeRows;
+  for (int e = tid; e < kTreeRows * nfeat; e += kTreeThreads) {
+    const int r = e / nfeat, f = e % nfeat;
+    sx[f * kTreeRows + r] = row0 + r < n ? X[(row0 + r) * nfeat + f] : 0.0;
+  }
+  // a batch is 16 KB of values and 8 KB of links: two and one 16-byte loads each
+  double2 rt[2];
+  uint4 rm;
+  auto fetch = [&](int t0) {
+    const double2 *pt = reinterpret_cast<const double2 *>(thr + (int64_t)t0 * kTreeNodes);
+    rt[0] = pt[tid];
+    rt[1] = pt[tid + kTreeThreads];
+    rm = reinterpret_cast<const uint4 *>(meta + (int64_t)t0 * kTreeNodes)[tid];
+  };
+  static_assert(kTreeBatch * kTreeNodes == 4 * kTreeThreads, "one batch in three loads");
+  const int row = (wave & 1) * 64 + tid % 64, tree = wave / 2 * kTreeIlp;
+  double acc = base;
+  fetch(0);
+  for (int t0 = 0; t0 < ntrees; t0 += kTreeBatch) {
+    __syncthreads();
+    reinterpret_cast<double2 *>(sthr)[tid] = rt[0];
+    reinterpret_cast<double2 *>(sthr)[tid + kTreeThreads] = rt[1];
+    reinterpret_cast<uint4 *>(smeta)[tid] = rm;
+    __syncthreads();
+    if (t0 + kTreeBatch < ntrees) fetch(t0 + kTreeBatch);
+    int at[kTreeIlp];
+#pragma unroll
+    for (int k = 0; k < kTreeIlp; ++k) at[k] = (tree + k) * kTreeNodes;
+    bool walking = true;
+    while (__any(walking)) {
+      walking = false;
+      uint32_t m[kTreeIlp];
+      double v[kTreeIlp];
+#pragma unroll
+      for (int k = 0; k < kTreeIlp; ++k) {
+        m[k] = smeta[at[k]];
+        v[k] = sthr[at[k]];
+      }
+#pragma unroll
+      for (int k = 0; k < kTreeIlp; ++k) {
+        const double x = sx[(m[k] >> 16 & (kTreeFeat - 1)) * kTreeRows + row];
+        const int next = (tree + k) * kTreeNodes + (x <= v[k] ? m[k] & 255 : m[k] >> 8 & 255);
+        const bool inner = !(m[k] & kTreeLeaf);
+        at[k] = inner ? next : at[k];
+        walking |= inner;
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < kTreeIlp; ++k) leaf[(tree + k) * kTreeRows + row] = sthr[at[k]];
+    __syncthreads();
+    if (tid < kTreeRows) {
+      const int nt = ntrees - t0 < kTreeBatch ? ntrees - t0 : kTreeBatch;
+      if (nt == kTreeBatch) {
+#pragma unroll
+        for (int k = 0; k < kTreeBatch; ++k) acc += leaf[k * kTreeRows + tid];
+      } else {
+        for (int k = 0; k < nt; ++k) acc += leaf[k * kTreeRows + tid];
+      }
+    }
+  }
+  if (tid < kTreeRows && row0 + tid < n) out[row0 + tid] = acc;
+}
+
+// Any trees: one thread per row, trees and features from memory.
 __global__ void forest_predict_kernel(const FNode *__restrict__ nodes,
                                       const int32_t *__restrict__ roots, int ntrees, double base,
                                       const double *__restrict__ X, int64_t n, int nfeat,
@@ -251,8 +338,10 @@ struct fdadi_forest {
   int ntrees = 0, nfeat = 0;
   int64_t nnodes = 0;
   double base = 0.0;
-  FNode *d_nodes = nullptr;
+  FNode *d_nodes = nullptr;     // any trees
   int32_t *d_roots = nullptr;
+  double *d_thr = nullptr;      // or small ones, in the tile kernel's layout
+  uint32_t *d_meta = nullptr;
 };
 
 extern "C" {
@@ -295,16 +384,37 @@ int fdadi_forest_create(int32_t ntrees, const int64_t *tree_start, int32_t nfeat
   f->nfeat = nfeat;
   f->nnodes = nn;
   f->base = base;
-  hipError_t e = hipMalloc((void **)&f->d_nodes, sizeof(FNode) * nn);
-  if (e == hipSuccess) e = hipMalloc((void **)&f->d_roots, sizeof(int32_t) * ntrees);
-  if (e == hipSuccess)
-    e = hipMemcpy(f->d_nodes, h.data(), sizeof(FNode) * nn, hipMemcpyHostToDevice);
-  if (e == hipSuccess)
-    e = hipMemcpy(f->d_roots, roots.data(), sizeof(int32_t) * ntrees, hipMemcpyHostToDevice);
+  hipError_t e = hipSuccess;
+  auto upload = [&](void **d, const void *src, size_t bytes) {
+    if (e == hipSuccess) e = hipMalloc(d, bytes);
+    if (e == hipSuccess) e = hipMemcpy(*d, src, bytes, hipMemcpyHostToDevice);
+  };
+  bool small = nfeat <= kTreeFeat;
+  for (int t = 0; t < ntrees; ++t) small = small && tree_start[t + 1] - tree_start[t] <= kTreeNodes;
+  if (small) {
+    const size_t slots =
+        (size_t)((ntrees + kTreeBatch - 1) / kTreeBatch) * kTreeBatch * kTreeNodes;
+    std::vector<double> thr(slots, 0.0);
+    std::vector<uint32_t> meta(slots, kTreeLeaf);
+    for (int t = 0; t < ntrees; ++t) {
+      const int64_t a = tree_start[t];
+      for (int64_t i = a; i < tree_start[t + 1]; ++i) {
+        const FNode &nd = h[(size_t)i];
+        const size_t s = (size_t)t * kTreeNodes + (size_t)(i - a);
+        thr[s] = nd.leaf ? nd.value : nd.thr;
+        if (!nd.leaf)
+          meta[s] = (uint32_t)nd.feature << 16 | (uint32_t)(nd.right - a) << 8 |
+                    (uint32_t)(nd.left - a);
+      }
+    }
+    upload((void **)&f->d_thr, thr.data(), sizeof(double) * slots);
+    upload((void **)&f->d_meta, meta.data(), sizeof(uint32_t) * slots);
+  } else {
+    upload((void **)&f->d_nodes, h.data(), sizeof(FNode) * nn);
+    upload((void **)&f->d_roots, roots.data(), sizeof(int32_t) * ntrees);
+  }
   if (e != hipSuccess) {
-    (void)hipFree(f->d_nodes);
-    (void)hipFree(f->d_roots);
-    delete f;
+    (void)fdadi_forest_destroy(f);
     set_error(std::string("fdadi_forest_create: ") + hipGetErrorString(e));
     return FDADI_ERR_HIP;
   }
@@ -316,6 +426,8 @@ int fdadi_forest_destroy(fdadi_forest *f) {
   if (!f) return FDADI_OK;
   (void)hipFree(f->d_nodes);
   (void)hipFree(f->d_roots);
+  (void)hipFree(f->d_thr);
+  (void)hipFree(f->d_meta);
   delete f;
   return FDADI_OK;
 }
@@ -325,6 +437,13 @@ int fdadi_forest_predict(const fdadi_forest *f, const double *d_X, int64_t n, do
   FDADI_REQUIRE(f && n >= 0 && (n == 0 || (d_X && d_out)), FDADI_ERR_ARG,
                 "fdadi_forest_predict: bad arguments");
   if (n == 0) return FDADI_OK;
+  if (f->d_thr) {
+    hipLaunchKernelGGL(forest_tile_kernel, dim3(grid_for(n, kTreeRows)), dim3(kTreeThreads), 0,
+                       as_stream(stream), f->d_thr, f->d_meta, f->ntrees, f->base, d_X, n,
+                       f->nfeat, d_out);
+    FDADI_CHECK_LAUNCH();
+    return FDADI_OK;
+  }
   hipLaunchKernelGGL(forest_predict_kernel, dim3(grid_for(n, 128)), dim3(128), 0,
                      as_stream(stream), f->d_nodes, f->d_roots, f->ntrees, f->base, d_X, n,
                      f->nfeat, d_out);
