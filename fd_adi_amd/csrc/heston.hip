@@ -426,17 +426,6 @@ __device__ __forceinline__ void load_lds16(const double *src, double *dst) {
 }
 __device__ __forceinline__ void lds_loads_done() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
-// 1 / d by two Newton steps from the hardware estimate (relative error
-// 2^-23, then 2^-46 and below 2^-90 before the last rounding): as the IEEE
-// division, whose special cases v_div_fixup supplies, at half its
-// instructions.
-__device__ __forceinline__ double recip(double d) {
-  double r = __builtin_amdgcn_rcp(d);
-  r = __builtin_fma(r, __builtin_fma(-d, r, 1.0), r);
-  r = __builtin_fma(r, __builtin_fma(-d, r, 1.0), r);
-  return __builtin_amdgcn_div_fixup(r, d, 1.0);
-}
-
 // Value of the lane before / after / two before within the tile's lanes
 // (quad_perm for four columns; row_shr / row_shl within a DPP row of 16
 // lanes for 8 and 16; wave_shr / wave_shl across the two DPP rows of a

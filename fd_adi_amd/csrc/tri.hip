@@ -115,7 +115,7 @@ __global__ void tri_apply_kernel(TriView o, const double *__restrict__ x,
 // forward-substituted values stay in LDS where lines are short (KEEP);
 // otherwise they go to scratch (`cpg`) and v, chunk by chunk.  One wave for 64
 // lines, which staged 16 rows at a time before each stretch of the chain, took
-// 121 us for 151 lines of 81 and 212 us for 81 lines of 151 (13 and 19 now).
+// 121 us for 151 lines of 81 and 212 us for 81 lines of 151 (10 and 16 now).
 constexpr int kSolveLines = 8, kSolveChunk = 64, kSolveThreads = 256;
 constexpr int kSolvePer = kSolveLines * kSolveChunk / kSolveThreads;  // elements per thread
 constexpr int kSolvePitch = kSolveChunk + 1;
@@ -230,7 +230,7 @@ tri_solve_kernel(TriView o, double *__restrict__ v, double *__restrict__ cpg) {
         k = 1;
       }
       auto eliminate = [&](double a, double b, double c, double d) {
-        const double m = 1.0 / (b - a * cprev);
+        const double m = recip(b - a * cprev);
         cprev = c * m;
         dprev = (d - a * dprev) * m;
       };
