@@ -946,7 +946,7 @@ __device__ __forceinline__ void spot_tiles(const Ctx &c, const Tile *__restrict_
       // I - tdt*A0 on this row (identity rows on Dirichlet rows and zero
       // off-diagonals at the line ends come from the bands), scaled by the
       // pivot.  The diagonal 1 - tdt*b is one fused operation, as
-      // spot_factor_kernel forms it, written out so that the compiler's
+      // spot_factor forms it, written out so that the compiler's
       // contraction choices cannot change how the recomputed pivots round.
       const double rd0 = recip(__builtin_fma(-tdt, B.mid, 1.0) - (-tsub * rdp) * cp);
       rdp = rd0;
@@ -1393,11 +1393,10 @@ __global__ void var_tables_kernel(const HOpt *opts, const int64_t *row_opt,
 // results.  One thread per option, loading as it went, took 224 us for
 // one option of 1,024 rows (57 now) and 33 us for 150 (12 now).
 constexpr int kFactorRows = 64;
-__global__ void __launch_bounds__(64) var_factor_kernel(HOpt *opts,
-                                                        const double *__restrict__ vars, double *vt,
-                                                        int64_t vt_n) {
-  __shared__ __attribute__((aligned(16))) double rows[kFactorRows][4];
-  const int k = blockIdx.x, lane = threadIdx.x;
+__device__ __forceinline__ void var_factor(double (*rows)[8], int k, HOpt *opts,
+                                           const double *__restrict__ vars, double *vt,
+                                           int64_t vt_n) {
+  const int lane = threadIdx.x;
   HOpt o = opts[k];
   const int64_t n = o.nv;
   const double *m = vars + o.vo;
@@ -1454,7 +1453,11 @@ __global__ void __launch_bounds__(64) var_factor_kernel(HOpt *opts,
       N[j] = -c * rd;
     }
   }
-  if (lane == 0) opts[k] = o;
+  if (lane == 0) {
+    opts[k].Gz = o.Gz;
+    opts[k].fold_f = o.fold_f;
+    opts[k].rdS0 = o.rdS0;
+  }
 }
 
 // Pivots 1/b' of I - tdt*A0 on every spot line, one wave per 64 lines of an
@@ -1463,10 +1466,8 @@ __global__ void __launch_bounds__(64) var_factor_kernel(HOpt *opts,
 // chunk ahead of the chain and read back from LDS, and the next rows' band
 // entries fill the chain's gaps.  Loading each row where it is used took 669
 // us on 2,048 x 1,024 nodes (212 now) and 50 us on 150 x 150 (17 now).
-__global__ void __launch_bounds__(64) spot_factor_kernel(Ctx c, const Tile *__restrict__ tiles,
-                                                         double *rd0) {
-  __shared__ __attribute__((aligned(16))) double rows[kFactorRows][8];
-  const Tile t = tiles[blockIdx.x];
+__device__ __forceinline__ void spot_factor(double (*rows)[8], const Ctx &c, Tile t,
+                                            double *rd0) {
   const HOpt o = c.opts[t.opt];
   const int lane = threadIdx.x;
   const int64_t j = t.start + lane, n = o.nS;
@@ -1512,6 +1513,19 @@ __global__ void __launch_bounds__(64) spot_factor_kernel(Ctx c, const Tile *__re
     }
   }
   if (o.barrier && in) rd[(n - 1) * o.nv] = 1.0 / (1.0 - (0.0 * rdprev) * cprev);
+}
+
+// Both factorisations, which are independent, side by side: work-groups
+// [0, nopt) the options' variance lines, the rest tiles of spot lines.  (Each
+// writes what the other does not read.)
+__global__ void __launch_bounds__(64) factor_kernel(Ctx c, HOpt *opts, int nopt,
+                                                    const double *__restrict__ vars, double *vt,
+                                                    const Tile *__restrict__ tiles, double *rd0) {
+  __shared__ __attribute__((aligned(16))) double rows[kFactorRows][8];
+  if ((int)blockIdx.x < nopt)
+    var_factor(rows, blockIdx.x, opts, vars, vt, c.vt_n);
+  else
+    spot_factor(rows, c, tiles[(int)blockIdx.x - nopt], rd0);
 }
 
 // Step sizes of every option from the scheme's theta and the dt multiplier,
@@ -2035,11 +2049,8 @@ int refactor(fdadi_hb *hb, hipStream_t s, const double *d_theta = nullptr,
                      hb->dt_scale, (int)(hb->scheme == FDADI_SCHEME_IMPLICIT),
                      reuse ? nullptr : hb->d_slots);
   FDADI_CHECK_LAUNCH();
-  hipLaunchKernelGGL(var_factor_kernel, dim3(hb->nopt), dim3(64), 0, s, hb->d_opts, hb->d_vars,
-                     hb->d_vt, hb->vt_n);
-  FDADI_CHECK_LAUNCH();
-  hipLaunchKernelGGL(spot_factor_kernel, dim3(hb->nftiles), dim3(64), 0, s, ctx_of(hb),
-                     hb->d_ftiles, hb->d_rd0);
+  hipLaunchKernelGGL(factor_kernel, dim3(hb->nopt + hb->nftiles), dim3(64), 0, s, ctx_of(hb),
+                     hb->d_opts, hb->nopt, hb->d_vars, hb->d_vt, hb->d_ftiles, hb->d_rd0);
   FDADI_CHECK_LAUNCH();
   if (!dev && !capturing) FDADI_TRY_HIP(hipStreamSynchronize(s));
   return FDADI_OK;
