@@ -1465,14 +1465,16 @@ __device__ __forceinline__ void var_factor(double (*rows)[8], int k, HOpt *opts,
 // waves): the table rows, the same for all lanes, are fetched 64 at a time a
 // chunk ahead of the chain and read back from LDS, and the next rows' band
 // entries fill the chain's gaps.  Loading each row where it is used took 669
-// us on 2,048 x 1,024 nodes (212 now) and 50 us on 150 x 150 (17 now).
+// us on 2,048 x 1,024 nodes (166 now) and 50 us on 150 x 150 (15 now).
 __device__ __forceinline__ void spot_factor(double (*rows)[8], const Ctx &c, Tile t,
                                             double *rd0) {
   const HOpt o = c.opts[t.opt];
   const int lane = threadIdx.x;
-  const int64_t j = t.start + lane, n = o.nS;
-  const bool in = j < o.nv;
-  const double v = c.vt[VT_V * c.vt_n + o.vo + (in ? j : o.nv - 1)];
+  const int64_t n = o.nS;
+  // lanes past the last column repeat it (no branch around the stores, which
+  // would keep a row's arithmetic from filling the gaps of another's)
+  const int64_t j = t.start + lane < o.nv ? t.start + lane : o.nv - 1;
+  const double v = c.vt[VT_V * c.vt_n + o.vo + j];
   double *rd = rd0 + o.off + j;
   double f[7];
   auto fetch = [&](int64_t i) {  // table row i of this lane's (the last one beyond it)
@@ -1487,7 +1489,7 @@ __device__ __forceinline__ void spot_factor(double (*rows)[8], const Ctx &c, Til
   };
   // Row 0 is Dirichlet, and the last one of a barrier option: a = c = 0, b = 1.
   double rdprev = 1.0, cprev = 0.0;
-  if (in) rd[0] = 1.0;
+  rd[0] = 1.0;
   const int64_t last = o.barrier ? n - 1 : n;
   fetch(1 + lane);
   for (int64_t i0 = 1; i0 < last; i0 += kFactorRows) {
@@ -1503,7 +1505,7 @@ __device__ __forceinline__ void spot_factor(double (*rows)[8], const Ctx &c, Til
       const double b = 1.0 - o.tdt * band_add(w[2], w[3], c00);
       rdprev = recip(b - (a * rdprev) * cprev);
       cprev = -o.tdt * band_add(w[4], w[5], c00);
-      if (in) rd[(i0 + q) * o.nv] = rdprev;
+      rd[(i0 + q) * o.nv] = rdprev;
     };
     if (last - i0 >= kFactorRows) {
 #pragma unroll 8
@@ -1512,7 +1514,7 @@ __device__ __forceinline__ void spot_factor(double (*rows)[8], const Ctx &c, Til
       for (int q = 0; q < (int)(last - i0); ++q) step(q);
     }
   }
-  if (o.barrier && in) rd[(n - 1) * o.nv] = 1.0 / (1.0 - (0.0 * rdprev) * cprev);
+  if (o.barrier) rd[(n - 1) * o.nv] = 1.0 / (1.0 - (0.0 * rdprev) * cprev);
 }
 
 // Both factorisations, which are independent, side by side: work-groups
