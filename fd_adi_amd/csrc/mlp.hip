@@ -585,7 +585,8 @@ __device__ __forceinline__ f32x4 update4(const UpdateArgs &a, int64_t i, f32x4 g
   f32x4 p = *reinterpret_cast<const f32x4 *>(a.p + i);
   if (MODE != UPDATE_COPIES && write_g) *reinterpret_cast<f32x4 *>(a.g + i) = g;
   if (MODE == UPDATE_ADAM) {
-    f32x4 m = *reinterpret_cast<const f32x4 *>(a.m + i), v = *reinterpret_cast<const f32x4 *>(a.v + i);
+    f32x4 m = *reinterpret_cast<const f32x4 *>(a.m + i);
+    f32x4 v = *reinterpret_cast<const f32x4 *>(a.v + i);
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
       float mt = m[t], vt = v[t];
