@@ -316,16 +316,16 @@ __device__ __forceinline__ double quad_carry(double M, double E, double2 *tot) {
 // ---- spot sweep ---------------------------------------------------------------
 // One 128-byte row of per-node spot coefficients, built from the spot table
 // with the boundary handling folded in:
-// [psub' pmid psup' qsub' | qmid qsup' pr qr | S*wsub S*wmid S*wsup S^2 | S snz 0 0]
+// [psub' pmid psup' qsub' | qmid qsup' pr qr | S*wsub S*wmid S*wsup S^2 | (padding)]
 // (p*: first-derivative bands scaled by r S, with -r/2 on the diagonal; q*:
 // raw second-derivative weights, and qr the raw residual, to be scaled by
 // c00 = (1/2 v) S^2 in the kernel) where ' marks band entries zeroed when
 // they multiply a Dirichlet neighbour (row 0 for row 1; row nS-1 for row nS-2
 // under a barrier) -- the explicit apply forces those neighbours to 0, and in
 // the solve the coupling to a Dirichlet row (whose value is 0) contributes
-// nothing -- and snz = [S != 0].  Dirichlet rows have all-zero bands.  A sweep
-// reads the first twelve fields of a row; S and snz only at row 0 (the spot
-// mesh increases strictly from S >= 0, so only row 0 can have S = 0).
+// nothing.  Dirichlet rows have all-zero bands, so row 0 has no use for S^2 and
+// holds [S != 0] there (the spot mesh increases strictly from S >= 0, so only
+// row 0 can have S = 0; S^2 itself is 0 already for S below 1e-162).
 constexpr int kSpRow = 16;
 constexpr int kSpFields = 12;
 
@@ -847,7 +847,7 @@ __device__ __forceinline__ void spot_tiles(const Ctx &c, const Tile *__restrict_
     enter_row<MODE, NL, HALF, true>(q, expand_raw<NL>(ub, jj), expand_raw<NL>(yb, jj), ends, lc.last, wb);
     // the S = 0 line (row 0 when the mesh starts at 0): A1 keeps only the -r/2
     // of the split
-    if (s == 0 && (TAB_LDS ? tch[11] : spr[11]) == 0.0) zero_line<MODE, HALF>(q, wb);
+    if (s == 0 && (TAB_LDS ? tch[11] : spr[11]) == 0.0) zero_line<MODE, HALF>(q, wb);  // [S != 0]
     // the next tile (this one again after the last)
     const Geom gn = RUNS ? geom_of(on, start_n) : g;
     // byte offsets of the row the walk loads next (row s + 1 + PF + k at step
@@ -1317,7 +1317,7 @@ __global__ void spot_tables_kernel(const HOpt *opts, int nopt, const int64_t *ro
   col[SP_WSUP * sp_n] = ws[2];
   col[SP_S * sp_n] = S;
   // AoS row of the spot sweep (layout at kSpRow): neighbour-of-Dirichlet band
-  // entries zeroed, cross weights premultiplied by S, S^2, S, [S != 0] flag.
+  // entries zeroed, cross weights premultiplied by S, S^2 (row 0: [S != 0]).
   double *row = spr + g * 16;
   const bool zsub = i == 1;                       // row 0 is Dirichlet
   const bool zsup = o.barrier && i == n - 2;      // row n-1 is Dirichlet
@@ -1332,11 +1332,7 @@ __global__ void spot_tables_kernel(const HOpt *opts, int nopt, const int64_t *ro
   row[8] = S * ws[0];
   row[9] = S * ws[1];
   row[10] = S * ws[2];
-  row[11] = S * S;
-  row[12] = S;
-  row[13] = S != 0.0 ? 1.0 : 0.0;
-  row[14] = 0.0;
-  row[15] = 0.0;
+  row[11] = i > 0 ? S * S : (S != 0.0 ? 1.0 : 0.0);
 }
 
 // One thread per variance node: A1 rows for S != 0 lines and cross weights.
