@@ -38,13 +38,16 @@ void set_error(const std::string &msg);
 inline hipStream_t as_stream(void *s) { return reinterpret_cast<hipStream_t>(s); }
 
 // 1 / d by two Newton steps from the hardware estimate (relative error
-// 2^-23, then 2^-46 and below 2^-90 before the last rounding): as the IEEE
-// division, whose special cases v_div_fixup supplies, at half its
-// instructions.
+// 2^-23, then 2^-46 and below 2^-90 before the last rounding): the IEEE
+// division at half its instructions.  v_div_fixup supplies d's sign and the
+// results for zeros, infinities, NaN and |d| <= 2^-1024 (whose reciprocals
+// overflow).  For |d| just above that the estimate overflows and the
+// reciprocal does not, so the estimate is held to finite numbers.
 __device__ __forceinline__ double recip(double d) {
-  double r = __builtin_amdgcn_rcp(d);
-  r = __builtin_fma(r, __builtin_fma(-d, r, 1.0), r);
-  r = __builtin_fma(r, __builtin_fma(-d, r, 1.0), r);
+  const double ad = __builtin_fabs(d);
+  double r = __builtin_fmin(__builtin_amdgcn_rcp(ad), 0x1.fffffffffffffp1023);
+  r = __builtin_fma(r, __builtin_fma(-ad, r, 1.0), r);
+  r = __builtin_fma(r, __builtin_fma(-ad, r, 1.0), r);
   return __builtin_amdgcn_div_fixup(r, d, 1.0);
 }
 
