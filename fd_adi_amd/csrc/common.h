@@ -41,14 +41,22 @@ inline hipStream_t as_stream(void *s) { return reinterpret_cast<hipStream_t>(s);
 // 2^-23, then 2^-46 and below 2^-90 before the last rounding): the IEEE
 // division at half its instructions.  v_div_fixup supplies d's sign and the
 // results for zeros, infinities, NaN and |d| <= 2^-1024 (whose reciprocals
-// overflow).  For |d| just above that the estimate overflows and the
-// reciprocal does not, so the estimate is held to finite numbers.
+// overflow).  For |d| within 2^-23 above that the estimate overflows and the
+// reciprocal does not: recip_any holds the estimate to finite numbers, for
+// pivots of any size (the line solver's); recip gives an infinity there, for
+// those of I - theta dt A, whose diagonal starts from 1 (one instruction more
+// per row made the spot sweeps 1% longer).
+__device__ __forceinline__ double recip_from(double r, double d) {
+  r = __builtin_fma(r, __builtin_fma(-d, r, 1.0), r);
+  return __builtin_fma(r, __builtin_fma(-d, r, 1.0), r);
+}
 __device__ __forceinline__ double recip(double d) {
+  return __builtin_amdgcn_div_fixup(recip_from(__builtin_amdgcn_rcp(d), d), d, 1.0);
+}
+__device__ __forceinline__ double recip_any(double d) {
   const double ad = __builtin_fabs(d);
-  double r = __builtin_fmin(__builtin_amdgcn_rcp(ad), 0x1.fffffffffffffp1023);
-  r = __builtin_fma(r, __builtin_fma(-ad, r, 1.0), r);
-  r = __builtin_fma(r, __builtin_fma(-ad, r, 1.0), r);
-  return __builtin_amdgcn_div_fixup(r, d, 1.0);
+  const double r = __builtin_fmin(__builtin_amdgcn_rcp(ad), 0x1.fffffffffffffp1023);
+  return __builtin_amdgcn_div_fixup(recip_from(r, ad), d, 1.0);
 }
 
 inline unsigned grid_for(int64_t n, int block) {

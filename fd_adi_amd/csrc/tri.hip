@@ -230,7 +230,7 @@ tri_solve_kernel(TriView o, double *__restrict__ v, double *__restrict__ cpg) {
         k = 1;
       }
       auto eliminate = [&](double a, double b, double c, double d) {
-        const double m = recip(b - a * cprev);
+        const double m = recip_any(b - a * cprev);
         cprev = c * m;
         dprev = (d - a * dprev) * m;
       };
