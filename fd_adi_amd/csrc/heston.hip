@@ -754,13 +754,20 @@ __device__ __forceinline__ void spot_tiles(const Ctx &c, const Tile *__restrict_
   // the grid repeat the last one, whose results are discarded)
   constexpr int UNITS = TPL * MAXL * kSpFields / 2;
   static_assert(!TAB_LDS || UNITS % 64 == 0, "whole waves of table units");
+  // The units' places are formed anew for each tile: left to itself the compiler
+  // keeps them (12 on 8-column tiles) in registers throughout the walk, which
+  // then spills (up to 70 registers on chunks of 16 rows: the second stages of
+  // HV and MCS on 512 grids of 512 x 128 in 8-column tiles took 450 us, 341 now;
+  // 425 and 420 with one tile per work-group).
   auto load_table = [&](const Geom &g, const OptWords &w) {
     const double *spr = c.spr + w.so() * kSpRow;
+    int tq = tid;
+    asm volatile("" : "+v"(tq));
     const int wave0 = __builtin_amdgcn_readfirstlane(tid / 64 * 64);
 #pragma unroll
     for (int e0 = 0; e0 < UNITS; e0 += THREADS) {
       if (UNITS % THREADS == 0 || e0 + wave0 < UNITS) {
-        const int e = e0 + tid, slot = e / 6, part = e % 6;
+        const int e = e0 + tq, slot = e / 6, part = e % 6;
         const int r = (slot / MAXL) * g.L + slot % MAXL;
         load_lds16(spr + (unsigned)((r < g.nS ? r : g.nS - 1) * kSpRow + part * 2),
                    tab + 2 * (e0 + wave0));
