@@ -1098,8 +1098,16 @@ __device__ __forceinline__ void spot_tiles(const Ctx &c, const Tile *__restrict_
   }
 }
 
+// Waves per SIMD that a sweep's registers have to leave room for.  Craig-Sneyd's
+// second stage on four-column tiles of 8 rows fits three (168 registers; left
+// alone it takes 170 and two): 1,024 uneven grids in 658 us instead of 739,
+// 512 grids of 512 x 128 in 335 instead of 389.
+constexpr int spot_waves(int mode, int threads, int nl, int maxl) {
+  return nl == 4 && maxl == 8 && mode == SM_CS ? 3 : threads == 256 ? 2 : 1;
+}
+
 template <int MODE, int THREADS, int NL, int MAXL>
-__global__ void __launch_bounds__(THREADS, THREADS == 256 ? 2 : 1)
+__global__ void __launch_bounds__(THREADS, spot_waves(MODE, THREADS, NL, MAXL))
 spot_sweep_kernel(Ctx c, const Tile *__restrict__ tiles, int ntiles, const double *__restrict__ U,
                   const double *__restrict__ Y, double *__restrict__ out) {
   extern __shared__ double lds[];

@@ -1,6 +1,7 @@
 """What the compiled kernels need, from the metadata of the code objects in the
 built library: the sweeps and factorisations keep everything in registers (no
-scratch memory per lane)."""
+scratch memory per lane), and the small sweeps leave room for three waves per
+SIMD (168 of its 512 registers each, in steps of eight)."""
 
 import os
 import struct
@@ -56,3 +57,10 @@ def test_no_scratch(name, least):
     bad = {n: (k[".private_segment_fixed_size"], k[".vgpr_spill_count"]) for n, k in ks.items()
            if k[".private_segment_fixed_size"] or k[".vgpr_spill_count"]}
     assert not bad
+
+
+@pytest.mark.parametrize("mode", [0, 2])  # SM_FIRST and SM_CS, four columns, 8 rows
+def test_three_waves(mode):
+    ks = {n: k[".vgpr_count"] for n, k in kernels().items()
+          if "spot_sweep_kernelILi%dE" % mode in n and "ELi4ELi8EEE" in n}
+    assert len(ks) == 4 and max(ks.values()) <= 168, ks
