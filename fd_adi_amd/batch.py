@@ -144,27 +144,38 @@ class HestonBatch(object):
         """Pick the fastest launch shape of each sweep kind for the configured
         scheme: every valid candidate is timed over ``steps`` steps with HIP
         events (the stage slots of that kind summed); the state is saved and
-        restored.  Returns {kind: (threads, lines)} as set."""
+        restored, and if a step fails the shapes are too.  Returns
+        {kind: (threads, lines)} as set."""
         if self.scheme is None:
             raise RuntimeError("autotune: configure the engine first")
         # stage slots of each kind in a step (fdadi_hb_step's launch order)
         order = {0: (1, 0), 1: (0, 1)}.get(self.scheme, (0, 1, 0, 1))
         saved = self.state_view().copy(True)
+        shapes = (self.get_shape(0), (self.get_shape(1)[0], 0))
         best = {}
-        for kind in (0, 1):
-            timings = []
-            for c in self.SHAPES[kind]:
-                try:
-                    self.set_shape(kind, *c)
-                except (ValueError, NotImplementedError):
-                    continue
-                self.step_timed(1)
-                st = self.step_timed(steps)
-                timings.append((sum(t for t, k in zip(st, order) if k == kind), c))
-            best[kind] = min(timings)[1]
-            self.set_shape(kind, *best[kind])
-        self.state_view().copy_from(saved)
-        self.sync()
+        try:
+            for kind in (0, 1):
+                timings = []
+                for c in self.SHAPES[kind]:
+                    # set_shape refuses shapes too small for the grids, a step
+                    # those whose tiles exceed the LDS in the scheme's stages
+                    # (8 columns of 513 to 1,024 rows; the implicit scheme's fit)
+                    try:
+                        self.set_shape(kind, *c)
+                        self.step_timed(1)
+                    except (ValueError, NotImplementedError):
+                        continue
+                    st = self.step_timed(steps)
+                    timings.append((sum(t for t, k in zip(st, order) if k == kind), c))
+                best[kind] = min(timings)[1]
+                self.set_shape(kind, *best[kind])
+        except BaseException:
+            for kind, c in enumerate(shapes):
+                self.set_shape(kind, *c)
+            raise
+        finally:
+            self.state_view().copy_from(saved)
+            self.sync()
         return best
 
     def get_shape(self, kind):
