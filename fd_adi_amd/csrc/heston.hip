@@ -1815,10 +1815,12 @@ int build_spot_tiles(fdadi_hb *hb) {
   return FDADI_OK;
 }
 
+constexpr size_t kCuLds = 160 * 1024;
+
 // Kernels using more than 64 KB of dynamic LDS must say so once.
 int allow_lds(const void *fn, size_t bytes) {
   if (bytes <= 65536) return FDADI_OK;
-  FDADI_REQUIRE(bytes <= 160 * 1024, FDADI_ERR_UNSUPPORTED,
+  FDADI_REQUIRE(bytes <= kCuLds, FDADI_ERR_UNSUPPORTED,
                 "sweep tile needs " + std::to_string(bytes) + " bytes of LDS (> 160 KB)");
   FDADI_TRY_HIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes));
   return FDADI_OK;
@@ -1880,8 +1882,10 @@ int launch_spot_t(const fdadi_hb *hb, const fdadi_hb::SweepGroup &g, const doubl
   const size_t lds = sizeof(double) * (carry + ex + tab);
   FDADI_RET(allow_lds((const void *)spot_sweep_kernel<MODE, T, NL, ML>, lds));
   // wide tiles: as many work-groups as run at once (two of 256 threads or one
-  // of 512 per CU), each taking tile after tile
-  const int slots = NL == 4 ? g.ntiles : 256 * 512 / T;
+  // of 512 per CU, as the LDS allows: one of 88 KB on 8 columns of 16 rows,
+  // where the second half of 512 began after the first half's whole share,
+  // 1,024 uneven grids in 553 us a stage, 525 now), each taking tile after tile
+  const int slots = NL == 4 ? g.ntiles : 256 * std::min<int>(512 / T, kCuLds / lds);
   hipLaunchKernelGGL((spot_sweep_kernel<MODE, T, NL, ML>), dim3(std::min(g.ntiles, slots)),
                      dim3(T), lds, s, ctx_of(hb), hb->d_stiles + g.first, g.ntiles, U, Y, out);
   FDADI_CHECK_LAUNCH();
