@@ -694,6 +694,11 @@ __global__ void zero_kernel(float *p, int64_t n) {
   if (i < n) p[i] = 0.f;
 }
 
+__global__ void copy_kernel(const double *__restrict__ x, int64_t n, double *__restrict__ y) {
+  const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  if (i < n) y[i] = x[i];
+}
+
 }  // namespace
 }  // namespace fdadi
 
@@ -785,13 +790,13 @@ RowArgs row_args(const fdadi_mlp *m, const double *P, int64_t rows) {
   return a;
 }
 
-// Prices of n rows: one launch, no workspace.  One round of work-groups over
+// One launch for n rows.  One round of work-groups over
 // the 256 CUs where that is enough: 32 rows each up to 8,192 (22.7 us; 28.0
 // with 64), 64 up to 16,384 (31 us; 37 with 32, 39 with 48).  Beyond that two
 // work-groups of 48 rows share a CU, one's SiLU beside the other's products:
 // 99.8 us for 50,000 rows and 355 us for 200,000 (64 rows, one per CU: 110 and
 // 368; 128 rows: 100 and 361).
-int predict_rows(const fdadi_mlp *m, const double *d_P, int64_t n, double *d_out, hipStream_t s) {
+int launch_rows(const fdadi_mlp *m, const double *d_P, int64_t n, double *d_out, hipStream_t s) {
   RowArgs a = row_args(m, d_P, n);
   a.out = d_out;
   if (n <= 256 * 32)
@@ -807,7 +812,28 @@ int predict_rows(const fdadi_mlp *m, const double *d_P, int64_t n, double *d_out
   return FDADI_OK;
 }
 
+// Prices of n rows, no workspace -- unless they are to lie in the features' own
+// memory: a work-group's prices would then overwrite rows that others have yet
+// to read, so they go to the row kernel's sums first (1,282 prices' room per 32
+// rows of the capacity: 5,128 at least), part by part.
+int predict_rows(const fdadi_mlp *m, const double *d_P, int64_t n, double *d_out, hipStream_t s) {
+  const uintptr_t p = reinterpret_cast<uintptr_t>(d_P), q = reinterpret_cast<uintptr_t>(d_out);
+  const bool apart = q + n * sizeof(double) <= p || p + n * m->n_in * sizeof(double) <= q;
+  if (apart) return launch_rows(m, d_P, n, d_out, s);
+  double *const tmp = reinterpret_cast<double *>(m->gpart);
+  const int64_t part = (int64_t)(m->max_rows / 32) * (kPart / 2);
+  for (int64_t r = 0; r < n; r += part) {
+    const int64_t rows = std::min(part, n - r);
+    FDADI_RET(launch_rows(m, d_P + r * m->n_in, rows, tmp, s));
+    hipLaunchKernelGGL(copy_kernel, dim3(grid_for(rows, 256)), dim3(256), 0, s, tmp, rows, d_out + r);
+    FDADI_CHECK_LAUNCH();
+  }
+  return FDADI_OK;
+}
+
+// Most rows of a call without allocation: callers split their batches by it.
 constexpr int kNoAllocRows = 4096;
+static_assert(kNoAllocRows <= kTile / 32 * (kPart / 2), "one part at the smallest capacity");
 
 }  // namespace
 }  // namespace fdadi

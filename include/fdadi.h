@@ -310,10 +310,12 @@ int fdadi_mlp_grad(fdadi_mlp *m, const double *d_P, const double *d_T, const int
 int fdadi_mlp_train_step(fdadi_mlp *m, const double *d_P, const double *d_T, const int *d_idx,
                          int32_t rows, float lr, void *stream);
 int fdadi_mlp_loss(const fdadi_mlp *m, float *loss);
-/* Prices for d_P [n x 8] into d_out [n]. */
+/* Prices for d_P [n x 8] into d_out [n], which may lie in d_P's memory: anywhere
+ * for as many rows as the model's max_rows, at its start for more. */
 int fdadi_mlp_predict(fdadi_mlp *m, const double *d_P, int64_t n, double *d_out, void *stream);
 /* fdadi_mlp_predict for callers that must not allocate: one launch, no
- * workspace, nothing shared between calls.  At most 4096 rows per call
+ * workspace, nothing shared between calls (where d_out lies in d_P's memory:
+ * two, through the model's training buffers).  At most 4096 rows per call
  * (FDADI_ERR_ARG beyond; split the batch). */
 int fdadi_mlp_predict_noalloc(const fdadi_mlp *m, const double *d_P, int64_t n, double *d_out,
                               void *stream);
