@@ -37,6 +37,9 @@ constexpr int kTreeNodes = 128, kTreeFeat = 16, kTreeBatch = 16, kTreeRows = 128
 constexpr int kTreeThreads = 512, kTreeIlp = 4;
 constexpr uint32_t kTreeLeaf = 0x80000000u;  // else feature << 16 | right << 8 | left
 static_assert(kTreeBatch == kTreeIlp * (kTreeThreads / 64) / (kTreeRows / 64), "waves' trees");
+// A tree takes 1.5 KB whatever its size; millions of tiny ones, whose nodes take
+// 32 bytes each, keep the layout of any trees beyond 4 GB of it.
+constexpr int64_t kTileTrees = (int64_t(4) << 30) / (kTreeNodes * 12);
 
 // thr: kTreeNodes values per tree (a leaf's is its value), meta likewise; both
 // padded to whole batches with leaves.
@@ -389,7 +392,7 @@ int fdadi_forest_create(int32_t ntrees, const int64_t *tree_start, int32_t nfeat
     if (e == hipSuccess) e = hipMalloc(d, bytes);
     if (e == hipSuccess) e = hipMemcpy(*d, src, bytes, hipMemcpyHostToDevice);
   };
-  bool small = nfeat <= kTreeFeat;
+  bool small = nfeat <= kTreeFeat && ntrees <= kTileTrees;
   for (int t = 0; t < ntrees; ++t) small = small && tree_start[t + 1] - tree_start[t] <= kTreeNodes;
   if (small) {
     const size_t slots =
