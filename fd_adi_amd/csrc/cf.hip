@@ -159,14 +159,15 @@ __device__ inline double exp_(double x) {
   return ldexp(1.0 + __builtin_fma(r * r, horner(r, c), r), __double2loint(t));
 }
 
-// 1 / x for a normal x of ordinary size, by two Newton steps.
-__device__ inline double recip(double x) {
+// 1 / x for a normal x of ordinary size, by two Newton steps (zeros, infinities
+// and subnormal numbers are not looked after, as the pivots' recip does).
+__device__ inline double recip_(double x) {
   double y = __builtin_amdgcn_rcp(x);
   y = __builtin_fma(y, __builtin_fma(-x, y, 1.0), y);
   return __builtin_fma(y, __builtin_fma(-x, y, 1.0), y);
 }
 __device__ inline double div_(double a, double b) {
-  const double rb = recip(b), q = a * rb;
+  const double rb = recip_(b), q = a * rb;
   return __builtin_fma(__builtin_fma(-q, b, a), rb, q);
 }
 // log x = e ln 2 + 2 atanh((m - 1) / (m + 1)), x = 2^e m, m in [sqrt 1/2, sqrt 2)
@@ -235,7 +236,7 @@ __device__ inline double lewis_integrand(double u, const Lewis &o) {
   // of xi +- d the one without cancellation (Re d > 0, and Im d has the sign of
   // xr times Im xi), and the other from their product -s2 q
   const double br = o.xr + (o.xr >= 0.0 ? dr : -dr), bi = xi + (o.xr >= 0.0 ? di : -di);
-  const double p = -(o.s2 * q) * recip(br * br + bi * bi), sr = p * br, si = -(p * bi);
+  const double p = -(o.s2 * q) * recip_(br * br + bi * bi), sr = p * br, si = -(p * bi);
   const double xpr = o.xr >= 0.0 ? br : sr, xpi = o.xr >= 0.0 ? bi : si;
   const double xmr = o.xr >= 0.0 ? sr : br, xmi = o.xr >= 0.0 ? si : bi;
   double s, c;
@@ -245,7 +246,7 @@ __device__ inline double lewis_integrand(double u, const Lewis &o) {
   const double nn = Nr * Nr + Ni * Ni;
   const double lr = log_(0.25 * (nn * rm));  // twice the logarithm's real part
   const double li = atan2_(Ni * dr - Nr * di, Nr * dr + Ni * di);
-  const double rq = recip(nn * q);  // 1 / nn = q rq, 1 / q = nn rq
+  const double rq = recip_(nn * q);  // 1 / nn = q rq, 1 / q = nn rq
   const double a1 = 1.0 - er, f = -(q * o.v0) * (q * rq);
   const double zr = o.kts * (xmr * o.T - lr) + f * (a1 * Nr - ei * Ni);
   const double zi = o.kts * (xmi * o.T - 2.0 * li) - f * (a1 * Ni + ei * Nr) + u * o.k;

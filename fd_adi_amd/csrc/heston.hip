@@ -1280,10 +1280,6 @@ var_sweep_kernel(Ctx c, const Tile *__restrict__ tiles, const double *__restrict
 }
 
 // ---- set-up kernels ---------------------------------------------------------------
-struct SetupOpt {
-  int64_t nS, nv, so, vo;  // mesh / table offsets
-};
-
 // One thread per spot node of every option: the (0,) and (0,0) template rows
 // (with boundary rows) scaled by r*S and 1/2*S^2, and the cross weights.
 __global__ void spot_tables_kernel(const HOpt *opts, int nopt, const int64_t *row_opt,
@@ -1692,7 +1688,6 @@ struct fdadi_hb {
 namespace fdadi {
 namespace {
 
-constexpr int kNL = 8;     // variance sweep: rows per tile
 constexpr int kMAXL = 16;  // variance sweep: positions per thread
 constexpr int kMAXLs = 8;  // spot sweep: rows per thread
 constexpr int kMAXLs3 = 12;  // spot sweep, 16-column tiles chosen per option: rows per thread
@@ -1860,14 +1855,6 @@ int build_var_tiles(fdadi_hb *hb) {
                           hipMemcpyHostToDevice));
   hb->nvtiles = (int)vtl.size();
   return FDADI_OK;
-}
-
-int threads_for(int64_t n, int nl = kNL, int maxl = kMAXL) {
-  // Threads per workgroup so that each line's chunk fits MAXL registers.
-  const int64_t need = (n + maxl - 1) / maxl * nl;
-  int t = 64;
-  while (t < need && t < 1024) t *= 2;
-  return t;
 }
 
 template <int MODE, int T, int NL, int ML>
