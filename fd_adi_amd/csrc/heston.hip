@@ -18,8 +18,8 @@
 // second-order backward row (with its -2 band entry, folded) at vmax.
 //
 // Sweeps.  A spot sweep gives each workgroup (option, tile of NL variance
-// columns) pairs, one or, for wide tiles, one after another; a variance sweep one workgroup per (option, tile of NL spot
-// rows).  The tile's right-hand side is formed (fusing every explicit term of
+// columns) pairs, one or, for wide tiles, one after another; a variance sweep
+// one workgroup per (option, tile of NL spot rows).  The tile's right-hand side is formed (fusing every explicit term of
 // the stage) straight into LDS, the NL tridiagonal lines are solved in LDS,
 // and the stage output (fusing the next stage's explicit term) is written
 // back: one read of each input vector and one write per stage, no
@@ -601,18 +601,22 @@ __device__ __forceinline__ void pin(double x) { asm volatile("" ::"v"(x)); }
 // run side by side on one XCD because each row of a tile also touches the
 // lines of the tiles beside it: walking along an option instead (eight tiles
 // in a row) tripled the bytes fetched and was slower.  On 4,096 such grids the
-// first stage went from 834 to 628 us, the Craig-Sneyd second stage from 1,014
-// to 860 us (one 512-thread work-group per CU on 32 columns); what bounds them
-// now is the memory system: 2.4 and 3.6 GB move at 4.0 to 4.2 TB/s in row
-// segments of 128 to 256 bytes.  Fewer VALU instructions (80 down to 66 per
-// point) or more rows in flight no longer shorten them, and lines touched a
-// tile ahead are evicted from the 4 MB L2 before they are used.
+// first stage went from 811 to 605 us, the Craig-Sneyd second stage from 973
+// to 811 us (one 512-thread work-group per CU on 32 columns).  They move 2.4 and
+// 3.7 GB, 4.0 and 4.6 TB/s, in row segments of 128 to 256 bytes; the variance
+// stage, whose rows are whole, reaches 5.6 TB/s, and 256 such grids, whose
+// vectors the last-level cache nearly holds, take as long for each, so it is
+// the access pattern rather than HBM that they wait for.  A variant with 66
+// instead of 80 VALU instructions a point gained 3%, more rows in flight
+// nothing, and lines touched a tile ahead are evicted from the 4 MB L2 before
+// they are used.
 // Four-column tiles (few tiles, a work-group each) keep the one-tile form.
 //
 // With theta = 1/2 every entry of theta dt A is half the entry of dt A, exactly,
-// so one set of products serves both (HALF): the same bits with 20 fewer
-// registers, which is what lets the Craig-Sneyd stages keep two waves per SIMD
-// without spills.  Other thetas take the general form.
+// so one set of products serves both (HALF): the same bits, and 1 to 5% less
+// time on wide tiles.  Other thetas take the general form.  (Both stand in one
+// kernel, chosen by the option's record: a captured graph stays valid when
+// theta changes.)
 //
 // The row walk keeps a window of three rows (i-1, i, i+1) of what the stage
 // needs from U and Y2, the loads of rows i+2 and i+3 in flight, and forms the
@@ -634,6 +638,7 @@ __device__ __forceinline__ void pin(double x) { asm volatile("" ::"v"(x)); }
 // keeps them out of both chunk maps.  In the last chunk, rows past the grid
 // (i >= nS) have finite values and follow row nS - 1, whose super-diagonal is
 // zero (n = 0), so they do not reach any valid row either way.
+
 // An option's record as the lanes of a wave hold it (lane l: its l-th 8-byte
 // word), loaded a tile ahead with a vector load -- a scalar load in flight
 // would make every LDS read of the walk wait for it -- and read out with
@@ -754,15 +759,17 @@ __device__ __forceinline__ void spot_tiles(const Ctx &c, const Tile *__restrict_
   // the grid repeat the last one, whose results are discarded)
   constexpr int UNITS = TPL * MAXL * kSpFields / 2;
   static_assert(!TAB_LDS || UNITS % 64 == 0, "whole waves of table units");
-  // The units' places are formed anew for each tile: left to itself the compiler
-  // keeps them (12 on 8-column tiles) in registers throughout the walk, which
-  // then spills (up to 70 registers on chunks of 16 rows: the second stages of
-  // HV and MCS on 512 grids of 512 x 128 in 8-column tiles took 450 us, 341 now;
-  // 425 and 420 with one tile per work-group).
+  // Left to itself the compiler keeps the units' places (12 on 8-column tiles) in
+  // registers throughout the walk, which then spills where chunks are long (up
+  // to 70 registers: the second stages of HV and MCS on 512 grids of 512 x 128 in
+  // 8-column tiles took 450 us, 341 now; 425 and 420 with one tile per
+  // work-group).  There they are formed anew for each tile; where they fit they
+  // stay (3 VALU instructions a point less on 32 columns, 0.8% of the time).
+  constexpr bool PLACES_FIT = MAXL == 8 || (NL == 32 ? MODE != SM_HV : NL == 16 && !HAS_Y);
   auto load_table = [&](const Geom &g, const OptWords &w) {
     const double *spr = c.spr + w.so() * kSpRow;
     int tq = tid;
-    asm volatile("" : "+v"(tq));
+    if constexpr (!PLACES_FIT) asm volatile("" : "+v"(tq));
     const int wave0 = __builtin_amdgcn_readfirstlane(tid / 64 * 64);
 #pragma unroll
     for (int e0 = 0; e0 < UNITS; e0 += THREADS) {
