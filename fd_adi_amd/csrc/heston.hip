@@ -601,8 +601,8 @@ __device__ __forceinline__ void pin(double x) { asm volatile("" ::"v"(x)); }
 // run side by side on one XCD because each row of a tile also touches the
 // lines of the tiles beside it: walking along an option instead (eight tiles
 // in a row) tripled the bytes fetched and was slower.  On 4,096 such grids the
-// first stage went from 811 to 605 us, the Craig-Sneyd second stage from 973
-// to 811 us (one 512-thread work-group per CU on 32 columns).  They move 2.4 and
+// first stage went from 811 to 608 us, the Craig-Sneyd second stage from 973
+// to 810 us (one 512-thread work-group per CU on 32 columns).  They move 2.4 and
 // 3.7 GB, 4.0 and 4.6 TB/s, in row segments of 128 to 256 bytes; the variance
 // stage, whose rows are whole, reaches 5.6 TB/s, and 256 such grids, whose
 // vectors the last-level cache nearly holds, take as long for each, so it is
@@ -764,7 +764,7 @@ __device__ __forceinline__ void spot_tiles(const Ctx &c, const Tile *__restrict_
   // to 70 registers: the second stages of HV and MCS on 512 grids of 512 x 128 in
   // 8-column tiles took 450 us, 341 now; 425 and 420 with one tile per
   // work-group).  There they are formed anew for each tile; where they fit they
-  // stay (3 VALU instructions a point less on 32 columns, 0.8% of the time).
+  // stay (3 VALU instructions a point less on 32 columns, 0.3% of a solve).
   constexpr bool PLACES_FIT = MAXL == 8 || (NL == 32 ? MODE != SM_HV : NL == 16 && !HAS_Y);
   auto load_table = [&](const Geom &g, const OptWords &w) {
     const double *spr = c.spr + w.so() * kSpRow;
